@@ -6,19 +6,30 @@
 //
 // One lane per query.  A bound first (one descent to the nearer child at every level and
 // that leaf's triangles), then a depth-first BVH walk, nearer child first; a subtree is
-// skipped when a lower bound of the squared distance from the query to its (outward padded)
-// box, computed in FP32 (box_d2), exceeds the best squared distance so far.  The walk's
-// stack is the ray kernels' (rmh_trace.hpp): the top rows in LDS, deeper entries in private
-// memory; held in registers, the 32 entries and their distances took the kernel to 190
-// VGPRs (two waves per SIMD).  An unbounded search pushes a subtree at almost every level of
-// its first descent, so the stack is deeper than a ray's: 16 LDS rows (8 KB per wave; the
-// kernel's registers allow five waves per SIMD, which the 160 KB of LDS of a CU then just
-// holds).  The triangle's closest point (Ericson, Real-Time Collision Detection, 5.1.5:
-// Voronoi regions of the vertices, edges and face) and its distance are evaluated in FP64,
-// so the result is the FP64 nearest triangle; equal distances go to the lower global face
-// index.  Outputs per query (each pointer may be NULL): distance (FLT_MAX when nothing lies
-// within max_distance), closest point, unit face normal (not flipped), face id within its
-// mesh, geom id, object id (0xFFFFFFFF for none; point and normal NaN).
+// skipped when its (outward padded) box lies farther than the bound.  Everything in the walk
+// is FP32 with proven margins (rmh_closest_bounds.hpp): a triangle gives a lower and an upper
+// bound of its distance, the upper ones shrink the search, and the triangles whose lower
+// bound does not exceed it are listed.  The list (6 slots per lane in LDS, emptied when a
+// closer triangle outdates all of it) is evaluated in FP64 at the end, when all lanes are
+// there, or when it is full: the triangle's closest point (Ericson, Real-Time Collision
+// Detection, 5.1.5: Voronoi regions of the vertices, edges and face) and its distance, so the
+// result is the FP64 nearest triangle; equal distances go to the lower global face index.
+// Evaluated in the leaves, the FP64 code ran for nearly every triangle, for one or two lanes
+// of the wave each time (44 triangles per query on the terrain, 6.7 of them closer than what
+// was known; 1.6 evaluations now).  Outputs per query (each pointer may be NULL): distance
+// (FLT_MAX when nothing lies within max_distance), closest point, unit face normal (not
+// flipped), face id within its mesh, geom id, object id (0xFFFFFFFF for none; point and
+// normal NaN).
+//
+// The lanes of a wave walk nodes together until half of those still searching hold a leaf,
+// then test their leaves together (terrain, 1M queries, FP64 evaluation still in the leaves:
+// 1.95 ms; waiting for a third 2.03, a quarter 2.12, an eighth 2.38, for all of them 3.19;
+// node and leaf steps mixed in one loop, as at first, 2.93).  The walk is bound by its chain of
+// dependent node and triangle loads and by the spread of the work between the lanes (on the
+// terrain 72 nodes per query, 146 for a wave's slowest): 4M queries now take 4.4 ms instead
+// of 8.0, 1M 1.73 instead of 2.93, 1M between scattered objects 1.22 instead of 1.72.  The
+// walk's stack is the ray kernels' (rmh_trace.hpp): the top rows in LDS, deeper entries in
+// private memory.
 //
 // Lanes of a wave that walk unrelated parts of the tree fetch its nodes separately: random
 // query sets fetch about 3x the node bytes of the same points in spatial order.  Batches of
@@ -31,6 +42,7 @@
 // or when the scratch cannot be had, the batch is walked in the caller's order.  The scratch
 // (17 B per query) comes from a pool of the library's own that keeps kPoolKeep bytes per
 // device between calls.
+#include "rmh_closest_bounds.hpp"
 #include "rmh_trace.hpp"
 
 #include <rocprim/device/device_radix_sort.hpp>
@@ -72,46 +84,78 @@ __device__ D3 closest_on_triangle(const D3& p, const D3& a, const D3& b, const D
   return madd(madd(a, ab, vb * den), ac, vc * den);
 }
 
-// A lower bound of the squared distance from the query (qx, qy, qz: FP32, as given) to the
-// box [lo, hi], in FP32: each difference of two floats is rounded once (relative error at
-// most 2^-24), the squares and the sum add three more roundings, so shrinking the result by
-// 2^-20 bounds it from below; an overflow to infinity is clamped to FLT_MAX (still below any
-// FP64 bound the walk can hold for such a box).  Pruning with a lower bound never drops a
-// box that holds the nearest point; the triangle distances stay FP64.
-__device__ __forceinline__ double box_d2(float qx, float qy, float qz, float lox, float hix, float loy, float hiy,
-                                         float loz, float hiz) {
-  const float dx = fmaxf(fmaxf(lox - qx, qx - hix), 0.0f);
-  const float dy = fmaxf(fmaxf(loy - qy, qy - hiy), 0.0f);
-  const float dz = fmaxf(fmaxf(loz - qz, qz - hiz), 0.0f);
-  const float d2 = (dx * dx + dy * dy + dz * dz) * (1.0f - 0x1p-20f);
-  return static_cast<double>(fminf(d2, FLT_MAX));
-}
-
 struct CPArgs {
   MapData map;
   const rmh_vec3* q;
   const uint32_t* order;  // lane i takes query order[i] when the spread test below holds
   const float* spread;    // summed wave extents of a sample: [0] caller's order, [1] sorted
   uint32_t n;
+  uint32_t per_wave;      // queries per wave, one lane each
   double best0;  // max_distance^2: a result needs d^2 < best0
   rmh_closest_outputs out;
 };
 
-constexpr int kClosestLds = 16;
+// 12 LDS stack rows and 6 candidate slots (7.5 KB per wave) keep the five waves per SIMD that
+// the registers allow (terrain, 1M queries: 1.70 ms; 10 rows 1.79, 16 rows and four waves 1.98;
+// 4 slots 1.72 there but 1.48 instead of 1.29 ms between scattered objects, where the list
+// overflows more often; 8 slots 1.77).
+constexpr int kClosestLds = 12;
+constexpr uint32_t kCand = 6;
+// Waves of consecutive queries are dealt to the XCDs 64 at a time, so that an XCD's L2 keeps a
+// region's nodes and triangles (contiguous ranges per XCD: terrain 1.70 ms against 1.73, but a
+// room, whose regions differ in cost, 0.43 ms against 0.39; round-robin waves 1.87 and 0.39).
+constexpr uint32_t kDealt = 64;
+// One lane per query, 64 queries per wave, or fewer while that leaves at most 3 waves per
+// SIMD: with the chip that empty, a wave's walk is as long as its slowest query's and its
+// loads touch fewer lines (1,000 queries on the terrain: 64 per wave 366 us, 1 per wave 290;
+// 16,000: 574, 8 per wave 496; 60,000: 551, 32 per wave 541; at 4 waves per SIMD 60,000
+// queries in a room took 112 us instead of 102).
+constexpr uint32_t kSparseWaves = 3072;
 constexpr float kSpreadRatio = 4.0f;
 
+// FP32 value at least the squared distance d2 (infinite for those beyond FP32).
+__device__ __forceinline__ float upper_f32(double d2) { return __double2float_ru(d2); }
+
 template <int STACK>
-__global__ __launch_bounds__(64, 4) void k_closest(const CPArgs a) {
+__global__ __launch_bounds__(64, 5) void k_closest(const CPArgs a) {
   __shared__ int2 stk[kClosestLds][64];
-  const uint32_t lane_q = blockIdx.x * 64 + threadIdx.x;
-  if (lane_q >= a.n) return;
+  __shared__ uint32_t cand[kCand][64];
+  const uint32_t lane_q = xcd_dealt<kDealt>(blockIdx.x, gridDim.x) * a.per_wave + threadIdx.x;
+  if (threadIdx.x >= a.per_wave || lane_q >= a.n) return;
   const bool reorder = a.order && a.spread[1] * kSpreadRatio < a.spread[0];
   const uint32_t i = reorder ? a.order[lane_q] : lane_q;
   const rmh_vec3 qv = a.q[i];
-  const D3 q = d3(qv.x, qv.y, qv.z);
+  const F3 qf{qv.x, qv.y, qv.z};
+  // The walk runs on FP32 bounds: `upper` is at least the smallest squared distance met so
+  // far (and at most about best0), and the triangles that may hold it are listed in LDS
+  // (`cand`), to be evaluated in FP64 together at the end, or when the list is full.  A
+  // triangle is dropped only when its lower bound exceeds `upper`, so every triangle at the
+  // smallest FP64 distance is evaluated.
   double best = a.best0;
   uint32_t best_slot = 0xFFFFFFFFu, best_face = 0xFFFFFFFFu;
-  D3 best_p = d3(0, 0, 0);
+  float upper = upper_f32(best);
+  float bound = walk_bound(upper);      // boxes beyond it hold nothing nearer
+  float least = __builtin_inff();       // least lower bound of the listed triangles
+  uint32_t n_cand = 0;
+  auto evaluate = [&]() {
+    const D3 q = d3(qv.x, qv.y, qv.z);
+    for (uint32_t k = 0; k < n_cand; k++) {
+      const uint32_t slot = cand[k][threadIdx.x];
+      const size_t s = static_cast<size_t>(slot) * 3;
+      const float4 v0 = a.map.tris[s], v1 = a.map.tris[s + 1], v2 = a.map.tris[s + 2];
+      const D3 p = closest_on_triangle(q, d3(v0.x, v0.y, v0.z), d3(v1.x, v1.y, v1.z), d3(v2.x, v2.y, v2.z));
+      const D3 dv = sub(p, q);
+      const double d2 = ddot(dv, dv);
+      const uint32_t face = __float_as_uint(v2.w);
+      if (d2 < best || (d2 == best && best_slot != 0xFFFFFFFFu && face < best_face)) {
+        best = d2;
+        best_slot = slot;
+        best_face = face;
+      }
+    }
+    n_cand = 0;
+    least = __builtin_inff();
+  };
   volatile int spill_mem[STACK > kClosestLds ? 2 * (STACK - kClosestLds) : 2];
   PrivInt* spill = (PrivInt*)spill_mem;
   int sp = 0;
@@ -122,17 +166,22 @@ __global__ __launch_bounds__(64, 4) void k_closest(const CPArgs a) {
     for (uint32_t k = 0; k < cnt; k++) {
       const size_t s = static_cast<size_t>(first + k) * 3;
       const float4 v0 = a.map.tris[s], v1 = a.map.tris[s + 1], v2 = a.map.tris[s + 2];
-      const D3 p = closest_on_triangle(q, d3(v0.x, v0.y, v0.z), d3(v1.x, v1.y, v1.z), d3(v2.x, v2.y, v2.z));
-      const D3 dv = sub(p, q);
-      const double d2 = ddot(dv, dv);
-      const uint32_t face = __float_as_uint(v2.w);
-      if (d2 < best || (d2 == best && best_slot != 0xFFFFFFFFu && face < best_face)) {
-        best = d2;
-        best_slot = first + k;
-        best_face = face;
-        best_p = p;
+      const D2Bounds d = triangle_bounds(fsub(F3{v0.x, v0.y, v0.z}, qf), fsub(F3{v1.x, v1.y, v1.z}, qf),
+                                         fsub(F3{v2.x, v2.y, v2.z}, qf));
+      if (d.lo > upper) continue;
+      if (d.hi < upper) {
+        upper = d.hi;
+        if (upper < least) { n_cand = 0; least = __builtin_inff(); }
       }
+      if (n_cand == kCand) {
+        evaluate();
+        upper = fminf(upper, upper_f32(best));
+      }
+      cand[n_cand][threadIdx.x] = first + k;
+      n_cand++;
+      least = fminf(least, d.lo);
     }
+    bound = walk_bound(upper);
   };
   int ref = kDone;
   if (a.map.n_faces) {
@@ -143,42 +192,54 @@ __global__ __launch_bounds__(64, 4) void k_closest(const CPArgs a) {
     int g = a.map.root;
     while (g >= 0) {
       const Node2 nd = a.map.nodes[g];
-      const double b0 = box_d2(qv.x, qv.y, qv.z, nd.a.x, nd.a.y, nd.a.z, nd.a.w, nd.c.x, nd.c.y);
-      const double b1 = box_d2(qv.x, qv.y, qv.z, nd.b.x, nd.b.y, nd.b.z, nd.b.w, nd.c.z, nd.c.w);
+      const float b0 = box_d2(qf, nd.a.x, nd.a.y, nd.a.z, nd.a.w, nd.c.x, nd.c.y);
+      const float b1 = box_d2(qf, nd.b.x, nd.b.y, nd.b.z, nd.b.w, nd.c.z, nd.c.w);
       g = b0 <= b1 ? nd.d.x : nd.d.y;
     }
     leaf_test(g);
+    n_cand = 0;  // the walk meets that leaf again
+    least = __builtin_inff();
     ref = a.map.root;
   }
-  while (ref != kDone) {
-    if (ref >= 0) {
-      const Node2 nd = a.map.nodes[ref];
-      const double b0 = box_d2(qv.x, qv.y, qv.z, nd.a.x, nd.a.y, nd.a.z, nd.a.w, nd.c.x, nd.c.y);
-      const double b1 = box_d2(qv.x, qv.y, qv.z, nd.b.x, nd.b.y, nd.b.z, nd.b.w, nd.c.z, nd.c.w);
-      const bool h0 = b0 <= best, h1 = b1 <= best;
-      if (h0 && h1) {
-        const bool first0 = b0 <= b1;
-        // one entry per level: the host picks STACK >= tree depth; the entry's distance is
-        // rounded down, so a pop never skips a box that could still hold the nearest point
-        push_ref<STACK, 64, kClosestLds, true>(stk, spill, sp, first0 ? nd.d.y : nd.d.x,
-                                               __double2float_rd(first0 ? b1 : b0));
-        ref = first0 ? nd.d.x : nd.d.y;
-        continue;
+  for (;;) {
+    for (;;) {
+      const uint64_t walking = __ballot(ref >= 0 && ref != kDone), holding = __ballot(ref < 0);
+      if (walking == 0 || 2 * __popcll(holding) >= __popcll(walking | holding)) break;
+      if (ref >= 0 && ref != kDone) {
+        const Node2 nd = a.map.nodes[ref];
+        const float b0 = box_d2(qf, nd.a.x, nd.a.y, nd.a.z, nd.a.w, nd.c.x, nd.c.y);
+        const float b1 = box_d2(qf, nd.b.x, nd.b.y, nd.b.z, nd.b.w, nd.c.z, nd.c.w);
+        const bool h0 = b0 <= bound, h1 = b1 <= bound;
+        if (h0 && h1) {
+          // one entry per level: the host picks STACK >= tree depth
+          const bool first0 = b0 <= b1;
+          push_ref<STACK, 64, kClosestLds, true>(stk, spill, sp, first0 ? nd.d.y : nd.d.x, first0 ? b1 : b0);
+          ref = first0 ? nd.d.x : nd.d.y;
+        } else if (h0) {
+          ref = nd.d.x;
+        } else if (h1) {
+          ref = nd.d.y;
+        } else {
+          ref = pop_ref<STACK, 64, kClosestLds, true>(stk, spill, sp, bound);
+        }
       }
-      if (h0) { ref = nd.d.x; continue; }
-      if (h1) { ref = nd.d.y; continue; }
-    } else {
-      leaf_test(ref);
     }
-    // pop the next subtree that can still hold something nearer: the bound rounded up to
-    // FP32 pops every entry with distance <= best (and at most a few more, whose children
-    // are tested again)
-    ref = pop_ref<STACK, 64, kClosestLds, true>(stk, spill, sp, __double2float_ru(best));
+    if (__ballot(ref < 0) == 0) break;
+    if (ref < 0) {
+      leaf_test(ref);
+      ref = pop_ref<STACK, 64, kClosestLds, true>(stk, spill, sp, bound);
+    }
   }
+  evaluate();
   const rmh_closest_outputs& o = a.out;
   if (best_slot != 0xFFFFFFFFu) {
     const size_t s = static_cast<size_t>(best_slot) * 3;
     const float4 nn = a.map.normals[best_slot];
+    D3 best_p = d3(0, 0, 0);
+    if (o.points) {  // evaluated again rather than held through the walk
+      const float4 v0 = a.map.tris[s], v1 = a.map.tris[s + 1], v2 = a.map.tris[s + 2];
+      best_p = closest_on_triangle(d3(qv.x, qv.y, qv.z), d3(v0.x, v0.y, v0.z), d3(v1.x, v1.y, v1.z), d3(v2.x, v2.y, v2.z));
+    }
     if (o.dist) o.dist[i] = static_cast<float>(sqrt(best));
     if (o.points) { rmh_vec3 v; v.x = (float)best_p.x; v.y = (float)best_p.y; v.z = (float)best_p.z; o.points[i] = v; }
     if (o.normals) { rmh_vec3 v; v.x = nn.x; v.y = nn.y; v.z = nn.z; o.normals[i] = v; }
@@ -362,7 +423,9 @@ extern "C" int rmh_closest_points(const rmh_map* map, const rmh_vec3* queries, u
   a.n = n;
   a.best0 = static_cast<double>(max_distance) * static_cast<double>(max_distance);
   a.out = *out;
-  const uint32_t blocks = (n + 63) / 64;
+  a.per_wave = 64;
+  while (a.per_wave > 1 && (n + a.per_wave / 2 - 1) / (a.per_wave / 2) <= kSparseWaves) a.per_wave /= 2;
+  const uint32_t blocks = (n + a.per_wave - 1) / a.per_wave;
   hipStream_t s = static_cast<hipStream_t>(stream);
   void* scratch = nullptr;
   a.spread = nullptr;

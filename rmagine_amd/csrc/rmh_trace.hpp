@@ -679,6 +679,18 @@ __device__ __forceinline__ uint32_t xcd_contiguous(uint32_t b, uint32_t n) {
   return xcd < r ? xcd * (q + 1) + idx : r * (q + 1) + (xcd - r) * q + idx;
 }
 
+// The same with ranges of S (a power of two) indices dealt to the XCDs in turn, each round
+// starting one XCD further, for work whose cost varies along the index: an XCD then gets a
+// share of every region.  What is left after the last full round is cut contiguously.  A
+// bijection on [0, n).
+template <uint32_t S>
+__device__ __forceinline__ uint32_t xcd_dealt(uint32_t b, uint32_t n) {
+  const uint32_t full = n & ~(8u * S - 1u);
+  if (b >= full) return full + xcd_contiguous(b - full, n - full);
+  const uint32_t idx = b >> 3, round = idx / S;
+  return (round * 8u + ((b + round) & 7u)) * S + (idx & (S - 1u));
+}
+
 // Most one-wave workgroups per launch of the (pose, tile) kernels: a dispatch holds the grid
 // size in work-items as a 32-bit count, so blocks x 64 stays below 2^31.
 constexpr uint64_t kMaxTileBlocks = 1ull << 25;
