@@ -24,9 +24,12 @@
 //       per-segment FP64 3x3 SVD (one-sided Jacobi) and the Umeyama rotation with the
 //       reflection fix (optimization.cpp:12-55, linalg.cu:1150-1190)
 //
-// Reductions are wave64 shuffles, then one LDS step across the waves of a block, then
-// (for segments split over several blocks) a second pass over the per-block partials in a
-// fixed order, so results are deterministic run to run.
+// Reductions are lane swaps and shuffles that halve the values a lane carries at each step,
+// then one LDS step across the waves of a block, then (for segments split over several
+// blocks) a second pass over the per-block partials, one block per segment, all in a fixed
+// order, so results are deterministic run to run.  Point-to-plane statistics of one
+// 131,072-point scan: 33 us of kernels with one butterfly per value, 64 blocks and one thread
+// per segment in the second pass, 10 us so; of one 16M-point cloud 540 and 170 us.
 #include "rmh_internal.hpp"
 
 #include <cmath>
@@ -167,31 +170,104 @@ struct Acc {
   double v[N];
 };
 
-template <int N>
-__device__ __forceinline__ void wave_sum(Acc<N>& a) {
-#pragma unroll
-  for (int k = 0; k < N; k++) {
-    double x = a.v[k];
-    for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
-    a.v[k] = x;
-  }
+// v and u of lanes 32 (or 16) apart, added crosswise: the lower of each pair gets the sum of
+// its own v and its partner's, the upper the sums of u (one swap instruction per word).
+__device__ __forceinline__ double swap_add32(double v, double u) {
+  const uint64_t a = __double_as_longlong(v), b = __double_as_longlong(u);
+  const auto lo = __builtin_amdgcn_permlane32_swap(static_cast<uint32_t>(a), static_cast<uint32_t>(b), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap(static_cast<uint32_t>(a >> 32), static_cast<uint32_t>(b >> 32), false, false);
+  return __hiloint2double(static_cast<int>(hi[0]), static_cast<int>(lo[0])) +
+         __hiloint2double(static_cast<int>(hi[1]), static_cast<int>(lo[1]));
 }
 
-// block-wide sum, result valid in thread 0
+__device__ __forceinline__ double swap_add16(double v, double u) {
+  const uint64_t a = __double_as_longlong(v), b = __double_as_longlong(u);
+  const auto lo = __builtin_amdgcn_permlane16_swap(static_cast<uint32_t>(a), static_cast<uint32_t>(b), false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap(static_cast<uint32_t>(a >> 32), static_cast<uint32_t>(b >> 32), false, false);
+  return __hiloint2double(static_cast<int>(hi[0]), static_cast<int>(lo[0])) +
+         __hiloint2double(static_cast<int>(hi[1]), static_cast<int>(lo[1]));
+}
+
+// The same for any lane distance OFF, by one exchange of the half a lane does not keep.
+template <int OFF>
+__device__ __forceinline__ double cross_add(double v, double u) {
+  const bool up = (threadIdx.x & OFF) != 0;
+  return (up ? u : v) + __shfl_xor(up ? v : u, OFF, 64);
+}
+
+// Sums of N values over the wave, each left in the lanes of one group (value g in lanes
+// [g 64 / P, (g + 1) 64 / P), P the power of two from N): every step halves the values a lane
+// carries, so 16 values take 17 exchanges instead of the 96 of one butterfly per value.
 template <int N>
-__device__ __forceinline__ void block_sum(Acc<N>& a, double (*lds)[N]) {
-  wave_sum(a);
+__device__ __forceinline__ double wave_sum(const Acc<N>& a) {
+  constexpr int P = N <= 16 ? 16 : 32;
+  double v[P / 2];
+#pragma unroll
+  for (int k = 0; k < P / 2; k++) v[k] = swap_add32(k < N ? a.v[k] : 0.0, k + P / 2 < N ? a.v[k + P / 2] : 0.0);
+#pragma unroll
+  for (int k = 0; k < P / 4; k++) v[k] = swap_add16(v[k], v[k + P / 4]);
+#pragma unroll
+  for (int k = 0; k < P / 8; k++) v[k] = cross_add<8>(v[k], v[k + P / 8]);
+#pragma unroll
+  for (int k = 0; k < P / 16; k++) v[k] = cross_add<4>(v[k], v[k + P / 16]);
+  double x;
+  if constexpr (P == 32) x = cross_add<2>(v[0], v[1]);
+  else x = v[0] + __shfl_xor(v[0], 2, 64);
+  return x + __shfl_xor(x, 1, 64);
+}
+
+// Block-wide sums: left in lds[0] (every thread may read them on return).
+template <int N>
+__device__ __forceinline__ void block_sum(const Acc<N>& a, double (*lds)[N]) {
+  constexpr int G = N <= 16 ? 4 : 2;  // lanes per value
+  const double x = wave_sum(a);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  if (lane == 0)
-    for (int k = 0; k < N; k++) lds[w][k] = a.v[k];
+  if (lane % G == 0 && lane / G < N) lds[w][lane / G] = x;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int k = 0; k < N; k++) {
-      double s = lds[0][k];
-      for (int j = 1; j < kWaves; j++) s += lds[j][k];
-      a.v[k] = s;
-    }
+  double s = 0.0;
+  if (threadIdx.x < N) {
+    s = lds[0][threadIdx.x];
+    for (int j = 1; j < kWaves; j++) s += lds[j][threadIdx.x];
   }
+  __syncthreads();
+  if (threadIdx.x < N) lds[0][threadIdx.x] = s;
+  __syncthreads();
+}
+
+// Block's sums of a segment split over several blocks.
+template <int N>
+__device__ __forceinline__ void store_partial(const double (*lds)[N], double* partial, uint64_t slot) {
+  if (threadIdx.x < N) partial[slot * N + threadIdx.x] = lds[0][threadIdx.x];
+}
+
+template <int N>
+__device__ __forceinline__ Acc<N> load_sums(const double (*lds)[N]) {
+  Acc<N> m;
+  for (int k = 0; k < N; k++) m.v[k] = lds[0][k];
+  return m;
+}
+
+// Sums of a segment's bps partials, left in lds[0]: one block per segment, its threads side by
+// side over the values and the partials (one thread per segment, walking all of them, took
+// 17 us for the 64 partials of one 131,072-point scan, more than the pass over its points).
+template <int N>
+__device__ __forceinline__ void combine_partials(const double* partial, uint32_t s, uint32_t bps, double (*lds)[N]) {
+  constexpr int P = N <= 16 ? 16 : 32, R = kBlk / P;  // R partials at a time
+  __shared__ double part[R][P];
+  const int k = threadIdx.x % P, r = threadIdx.x / P;
+  double x = 0.0;
+  if (k < N) {
+    const double* p = partial + static_cast<uint64_t>(s) * bps * N + k;
+#pragma unroll 4
+    for (uint32_t b = r; b < bps; b += R) x += p[static_cast<uint64_t>(b) * N];
+  }
+  part[r][k] = x;
+  __syncthreads();
+  if (threadIdx.x < N) {
+    for (int j = 1; j < R; j++) x += part[j][threadIdx.x];
+    lds[0][threadIdx.x] = x;
+  }
+  __syncthreads();
 }
 
 // moments: [0] count, [1..3] sum a, [4..6] sum b, [7..15] sum b_r a_c (column-major, c*3+r)
@@ -253,20 +329,14 @@ __global__ __launch_bounds__(kBlk) void k_moments(const MomArgs a) {
     acc_pair(m, x.x, x.y, x.z, y.x, y.y, y.z);
   }
   block_sum(m, lds);
-  if (threadIdx.x != 0) return;
-  if (a.bps == 1) finalize_moments(a, s, m);
-  else
-    for (int k = 0; k < kMom; k++) a.partial[(static_cast<uint64_t>(s) * a.bps + bb) * kMom + k] = m.v[k];
+  if (a.bps > 1) store_partial(lds, a.partial, static_cast<uint64_t>(s) * a.bps + bb);
+  else if (threadIdx.x == 0) finalize_moments(a, s, load_sums(lds));
 }
 
-__global__ void k_moments_combine(const MomArgs a) {
-  const uint32_t s = blockIdx.x * kBlk + threadIdx.x;
-  if (s >= a.nseg) return;
-  Acc<kMom> m;
-  zero(m);
-  for (uint32_t b = 0; b < a.bps; b++)
-    for (int k = 0; k < kMom; k++) m.v[k] += a.partial[(static_cast<uint64_t>(s) * a.bps + b) * kMom + k];
-  finalize_moments(a, s, m);
+__global__ __launch_bounds__(kBlk) void k_moments_combine(const MomArgs a) {
+  __shared__ double lds[1][kMom];
+  combine_partials(a.partial, blockIdx.x, a.bps, lds);
+  if (threadIdx.x == 0) finalize_moments(a, blockIdx.x, load_sums(lds));
 }
 
 // ---- correspondence statistics ------------------------------------------------------------
@@ -382,22 +452,18 @@ __global__ __launch_bounds__(kBlk) __attribute__((amdgpu_waves_per_eu(6))) void 
     acc_pair(m, dx, dy, dz, mx, my, mz);
   }
   block_sum(m, lds);
-  if (threadIdx.x != 0) return;
-  if (a.bps == 1) finalize_stats(&a.out[s], m, c);
-  else
-    for (int k = 0; k < kMom; k++) a.partial[(static_cast<uint64_t>(s) * a.bps + bb) * kMom + k] = m.v[k];
+  if (a.bps > 1) store_partial(lds, a.partial, static_cast<uint64_t>(s) * a.bps + bb);
+  else if (threadIdx.x == 0) finalize_stats(&a.out[s], load_sums(lds), c);
 }
 
-__global__ void k_stats_combine(const StatArgs a) {
-  const uint32_t s = blockIdx.x * kBlk + threadIdx.x;
-  if (s >= a.nseg) return;
+__global__ __launch_bounds__(kBlk) void k_stats_combine(const StatArgs a) {
+  __shared__ double lds[1][kMom];
+  const uint32_t s = blockIdx.x;
+  combine_partials(a.partial, s, a.bps, lds);
+  if (threadIdx.x != 0) return;
   const rmh_transform P = a.pre[a.npre == 1 ? 0 : s];
   const double c[3] = {(double)P.t.x, (double)P.t.y, (double)P.t.z};
-  Acc<kMom> m;
-  zero(m);
-  for (uint32_t b = 0; b < a.bps; b++)
-    for (int k = 0; k < kMom; k++) m.v[k] += a.partial[(static_cast<uint64_t>(s) * a.bps + b) * kMom + k];
-  finalize_stats(&a.out[s], m, c);
+  finalize_stats(&a.out[s], load_sums(lds), c);
 }
 
 // ---- objectwise point-to-plane statistics ---------------------------------------------------
@@ -474,7 +540,7 @@ __global__ __launch_bounds__(kBlk) void k_stats_objectwise(const ObjArgs a) {
     acc_pair(m, dx, dy, dz, dx + nn.x * spd, dy + nn.y * spd, dz + nn.z * spd);
   }
   block_sum(m, lds);
-  if (threadIdx.x == 0) finalize_stats(&a.out[o], m, c);
+  if (threadIdx.x == 0) finalize_stats(&a.out[o], load_sums(lds), c);
 }
 
 // ---- point-to-plane Gauss-Newton system -------------------------------------------------------
@@ -563,20 +629,14 @@ __global__ __launch_bounds__(kBlk) void k_p2l_system(const LinArgs a) {
     m.v[28] += w * r * r;
   }
   block_sum(m, lds);
-  if (threadIdx.x != 0) return;
-  if (a.bps == 1) finalize_system(&a.out[s], m);
-  else
-    for (int k = 0; k < kLin; k++) a.partial[(static_cast<uint64_t>(s) * a.bps + bb) * kLin + k] = m.v[k];
+  if (a.bps > 1) store_partial(lds, a.partial, static_cast<uint64_t>(s) * a.bps + bb);
+  else if (threadIdx.x == 0) finalize_system(&a.out[s], load_sums(lds));
 }
 
-__global__ void k_p2l_system_combine(const LinArgs a) {
-  const uint32_t s = blockIdx.x * kBlk + threadIdx.x;
-  if (s >= a.nseg) return;
-  Acc<kLin> m;
-  for (int k = 0; k < kLin; k++) m.v[k] = 0.0;
-  for (uint32_t b = 0; b < a.bps; b++)
-    for (int k = 0; k < kLin; k++) m.v[k] += a.partial[(static_cast<uint64_t>(s) * a.bps + b) * kLin + k];
-  finalize_system(&a.out[s], m);
+__global__ __launch_bounds__(kBlk) void k_p2l_system_combine(const LinArgs a) {
+  __shared__ double lds[1][kLin];
+  combine_partials(a.partial, blockIdx.x, a.bps, lds);
+  if (threadIdx.x == 0) finalize_system(&a.out[blockIdx.x], load_sums(lds));
 }
 
 // ---- Umeyama ------------------------------------------------------------------------------
@@ -761,13 +821,14 @@ __global__ void k_stats_pack(const rmh_vec3* ds, const rmh_vec3* ms, const float
 
 uint32_t blocks_per_segment(uint64_t seg, uint32_t nseg) {
   // enough blocks for several rounds of the chip's resident blocks (>= 8192 in total, so
-  // that the last, partly filled round is a small part of the launch), at least 2048
-  // elements per block
-  const uint64_t by_size = (seg + 2047) / 2048;
+  // that the last, partly filled round is a small part of the launch), at least 1024 elements
+  // per block (one scan of 131,072 points: 128 blocks), and at most 2048 per segment (eight
+  // blocks per CU for a single large segment; with 256, one wave per SIMD streamed it)
+  const uint64_t by_size = (seg + 1023) / 1024;
   const uint64_t want = (8192 + nseg - 1) / nseg;
   uint64_t b = want < by_size ? want : by_size;
   if (b < 1) b = 1;
-  if (b > 256) b = 256;
+  if (b > 2048) b = 2048;
   return static_cast<uint32_t>(b);
 }
 
@@ -871,7 +932,7 @@ int rmh_vec3_moments(const rmh_vec3* a, const rmh_vec3* b, const uint8_t* mask, 
   k_moments<<<dim3(A.bps, n_segments), kBlk, 0, stream>>>(A);
   RMH_HIP_TRY(hipGetLastError());
   if (A.bps > 1) {
-    k_moments_combine<<<grid1(n_segments), kBlk, 0, stream>>>(A);
+    k_moments_combine<<<n_segments, kBlk, 0, stream>>>(A);
     RMH_HIP_TRY(hipGetLastError());
     if (tmp.p) RMH_HIP_TRY(hipStreamSynchronize(stream));
   }
@@ -922,7 +983,7 @@ int stats_launch(const StatArgs& A, hipStream_t stream) {
     k_stats<uint64_t><<<dim3(A.bps, A.nseg), kBlk, 0, stream>>>(A);
   RMH_HIP_TRY(hipGetLastError());
   if (A.bps > 1) {
-    k_stats_combine<<<grid1(A.nseg), kBlk, 0, stream>>>(A);
+    k_stats_combine<<<A.nseg, kBlk, 0, stream>>>(A);
     RMH_HIP_TRY(hipGetLastError());
   }
   return RMH_OK;
@@ -1092,7 +1153,7 @@ int rmh_linear_system_p2l(const rmh_transform* pre_transforms, uint32_t n_pre, c
   k_p2l_system<<<dim3(A.bps, n_segments), kBlk, 0, stream>>>(A);
   RMH_HIP_TRY(hipGetLastError());
   if (A.bps > 1) {
-    k_p2l_system_combine<<<grid1(n_segments), kBlk, 0, stream>>>(A);
+    k_p2l_system_combine<<<n_segments, kBlk, 0, stream>>>(A);
     RMH_HIP_TRY(hipGetLastError());
     if (tmp.p) RMH_HIP_TRY(hipStreamSynchronize(stream));
   }
