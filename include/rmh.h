@@ -362,6 +362,15 @@ int rmh_pose_grad(const rmh_map* map, const rmh_sensor* sensor, const rmh_transf
                   const rmh_transform* Tbm_dev, uint32_t n_poses, const float* target_dev,
                   const uint8_t* target_mask_dev, int per_pose_targets, float huber_delta,
                   double* out_dev, void* workspace, size_t workspace_bytes, void* stream);
+/* The same loss of the poses (t0 + tau, Exp(omega) R0) for xi = (tau xyz, omega xyz), 6 doubles
+ * per pose, and its gradient with respect to xi: loss_dev one double, grad_dev 6 doubles per
+ * pose.  Poses, loss and gradient are formed on the device, in three launches.
+ * workspace: rmh_pose_loss_workspace_size bytes, or NULL as above. */
+int rmh_pose_loss_workspace_size(const rmh_map* map, const rmh_sensor* sensor, uint32_t n_poses, size_t* bytes);
+int rmh_pose_loss(const rmh_map* map, const rmh_sensor* sensor, const rmh_transform* Tsb,
+                  const rmh_transform* T0_dev, const double* xi_dev, uint32_t n_poses, const float* target_dev,
+                  const uint8_t* target_mask_dev, int per_pose_targets, float huber_delta,
+                  double* loss_dev, double* grad_dev, void* workspace, size_t workspace_bytes, void* stream);
 
 /* ---- math layer (rmagine_cuda's math, src/rmagine_cuda/src/math/) --------------------- */
 

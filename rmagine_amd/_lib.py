@@ -86,6 +86,9 @@ _SIGNATURES = {
     "rmh_pose_grad_workspace_size": (c_int, [c_void_p, c_void_p, c_u32, ctypes.POINTER(c_size)]),
     "rmh_pose_grad": (c_int, [c_void_p, c_void_p, ctypes.POINTER(T.rmh_transform), c_void_p, c_u32, c_void_p,
                               c_void_p, c_int, ctypes.c_float, c_void_p, c_void_p, c_size, c_void_p]),
+    "rmh_pose_loss_workspace_size": (c_int, [c_void_p, c_void_p, c_u32, ctypes.POINTER(c_size)]),
+    "rmh_pose_loss": (c_int, [c_void_p, c_void_p, ctypes.POINTER(T.rmh_transform), c_void_p, c_void_p, c_u32, c_void_p,
+                              c_void_p, c_int, ctypes.c_float, c_void_p, c_void_p, c_void_p, c_size, c_void_p]),
     "rmh_transform_set_identity": (c_int, [c_void_p, c_u32, c_void_p]),
     "rmh_transform_mul": (c_int, [c_void_p, c_u32, c_void_p, c_u32, c_void_p, c_u32, c_void_p]),
     "rmh_transform_inv": (c_int, [c_void_p, c_void_p, c_u32, c_void_p]),

@@ -33,13 +33,8 @@ def workspace_bytes(sim: SimulatorHip, n_poses: int) -> int:
     return n.value
 
 
-def pose_grad(sim: SimulatorHip, Tbm: torch.Tensor, target: torch.Tensor, target_mask: torch.Tensor | None = None,
-              per_pose_targets: bool = False, huber_delta: float = 0.05, out: torch.Tensor | None = None,
-              workspace: torch.Tensor | None = None, stream=None) -> torch.Tensor:
-    """Loss and gradient per pose: (N, 8) float64 {L, dL/dtau xyz, dL/domega xyz, rays used}.
-
-    Tbm: (N, 8) float32 device poses; target: (W*H,) or (N*W*H,) float32 device ranges.
-    """
+def _check_inputs(sim, Tbm, target, target_mask, per_pose_targets) -> int:
+    """What pose_grad asks of its arguments; the number of poses."""
     if sim.map() is None:
         raise _lib.NoMapError(3, "pose_grad: no map set")
     if sim._sensor is None:
@@ -52,6 +47,33 @@ def pose_grad(sim: SimulatorHip, Tbm: torch.Tensor, target: torch.Tensor, target
     need = rays * (N if per_pose_targets else 1)
     if target.numel() != need or (target_mask is not None and target_mask.numel() != need):
         raise ValueError(f"target (and mask) must hold {need} entries")
+    return N
+
+
+def _pose_loss(sim, T0, xi, target, target_mask, per_pose_targets, huber_delta):
+    """Loss (N,) and gradient (N, 6) of perturb(T0, xi) by rmh_pose_loss: three launches, where
+    forming the poses and applying the Jacobian in torch took about sixty."""
+    N = _check_inputs(sim, T0, target, target_mask, per_pose_targets)
+    n = ctypes.c_size_t()
+    _lib.call("rmh_pose_loss_workspace_size", sim.map().handle, sim._sensor.handle, N, ctypes.byref(n))
+    ws = torch.empty(n.value, dtype=torch.uint8, device=T0.device)
+    loss = torch.empty(N, dtype=torch.float64, device=T0.device)
+    grad = torch.empty((N, 6), dtype=torch.float64, device=T0.device)
+    Tsb = T.transform_to_c(sim._Tsb)
+    _lib.call("rmh_pose_loss", sim.map().handle, sim._sensor.handle, ctypes.byref(Tsb), _ptr(T0), _ptr(xi), N,
+              _ptr(target), _ptr(target_mask), int(bool(per_pose_targets)), float(huber_delta), _ptr(loss), _ptr(grad),
+              _ptr(ws), ws.numel(), stream_handle())
+    return loss, grad
+
+
+def pose_grad(sim: SimulatorHip, Tbm: torch.Tensor, target: torch.Tensor, target_mask: torch.Tensor | None = None,
+              per_pose_targets: bool = False, huber_delta: float = 0.05, out: torch.Tensor | None = None,
+              workspace: torch.Tensor | None = None, stream=None) -> torch.Tensor:
+    """Loss and gradient per pose: (N, 8) float64 {L, dL/dtau xyz, dL/domega xyz, rays used}.
+
+    Tbm: (N, 8) float32 device poses; target: (W*H,) or (N*W*H,) float32 device ranges.
+    """
+    N = _check_inputs(sim, Tbm, target, target_mask, per_pose_targets)
     if out is None:
         out = torch.empty((N, 8), dtype=torch.float64, device=Tbm.device)
     nbytes = workspace_bytes(sim, N)
@@ -114,16 +136,22 @@ class PoseRangeLoss(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, xi, T0, sim, target, target_mask=None, huber_delta=0.05):
-        Tp = perturb(T0, xi.detach())
-        res = pose_grad(sim, Tp, target, target_mask, per_pose_targets=target.numel() != sim._sensor.W * sim._sensor.H,
-                        huber_delta=huber_delta)
-        J = so3_left_jacobian(xi.detach().to(torch.float64)[:, 3:])
-        g = torch.empty((xi.shape[0], 6), dtype=torch.float64, device=xi.device)
-        g[:, :3] = res[:, 1:4]
-        g[:, 3:] = torch.einsum("nji,nj->ni", J, res[:, 4:7])
+        per_pose = target.numel() != sim._sensor.W * sim._sensor.H
+        if (xi.device.type == "cuda" and T0.device == xi.device and T0.dtype == torch.float32 and xi.shape[0] > 0
+                and xi.shape == (T0.shape[0], 6) and T0.shape == (xi.shape[0], 8)):
+            loss, g = _pose_loss(sim, T0.detach().contiguous(), xi.detach().to(torch.float64).contiguous(), target,
+                                 target_mask, per_pose, huber_delta)
+        else:
+            Tp = perturb(T0, xi.detach())
+            res = pose_grad(sim, Tp, target, target_mask, per_pose_targets=per_pose, huber_delta=huber_delta)
+            J = so3_left_jacobian(xi.detach().to(torch.float64)[:, 3:])
+            g = torch.empty((xi.shape[0], 6), dtype=torch.float64, device=xi.device)
+            g[:, :3] = res[:, 1:4]
+            g[:, 3:] = torch.einsum("nji,nj->ni", J, res[:, 4:7])
+            loss = res[:, 0]
         ctx.save_for_backward(g)
         ctx.xi_dtype = xi.dtype
-        return res[:, 0]
+        return loss
 
     @staticmethod
     def backward(ctx, grad_out):
