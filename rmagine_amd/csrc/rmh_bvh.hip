@@ -40,6 +40,7 @@ namespace {
 using namespace rmh;
 
 constexpr int kBlock = 256;
+constexpr uint32_t kWideBlocks = 2048;  // grid-stride passes: eight blocks per CU
 constexpr uint32_t kLeafBit = kTreeLeafBit;
 constexpr int kTreeletRounds = 3;
 // largest map: node references must stay below 2^26 (32-bit node byte offsets in the ray kernels)
@@ -71,34 +72,34 @@ __global__ void k_init(float* bounds, uint32_t* err) {
   else if (threadIdx.x == 6) *err = 0u;
 }
 
-// Step 1.
+// Step 1.  At most kWideBlocks blocks: the bounds' atomics go to six addresses, and with a
+// block per 256 faces they took most of its 0.33 ms on the 2.1M-triangle terrain.
 __global__ __launch_bounds__(kBlock) void k_prep(const float* __restrict__ V, uint32_t nv,
                                                  const uint32_t* __restrict__ F, uint32_t nf,
                                                  float4* __restrict__ lo, float4* __restrict__ hi,
                                                  float* bounds, uint32_t* err) {
-  const uint32_t f = blockIdx.x * kBlock + threadIdx.x;
   float cmin[3] = {FLT_MAX, FLT_MAX, FLT_MAX};
   float cmax[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
-  if (f < nf) {
+  uint32_t bad = 0;
+  for (uint32_t f = blockIdx.x * kBlock + threadIdx.x; f < nf; f += gridDim.x * kBlock) {
     uint32_t idx[3] = {F[3 * f + 0], F[3 * f + 1], F[3 * f + 2]};
-    bool bad = false;
     for (int k = 0; k < 3; k++) {
-      if (idx[k] >= nv) { bad = true; idx[k] = 0; }
+      if (idx[k] >= nv) { bad |= 1u; idx[k] = 0; }
     }
-    if (bad) atomicOr(err, 1u);
     float b0[3], b1[3];
     for (int a = 0; a < 3; a++) {
       const float x0 = V[3 * idx[0] + a], x1 = V[3 * idx[1] + a], x2 = V[3 * idx[2] + a];
       b0[a] = fminf(x0, fminf(x1, x2));
       b1[a] = fmaxf(x0, fmaxf(x1, x2));
-      if (!(isfinite(x0) && isfinite(x1) && isfinite(x2))) atomicOr(err, 2u);
+      if (!(isfinite(x0) && isfinite(x1) && isfinite(x2))) bad |= 2u;
       const float c = 0.5f * b0[a] + 0.5f * b1[a];
-      cmin[a] = c;
-      cmax[a] = c;
+      cmin[a] = fminf(cmin[a], c);
+      cmax[a] = fmaxf(cmax[a], c);
     }
     lo[f] = make_float4(b0[0], b0[1], b0[2], 0.0f);
     hi[f] = make_float4(b1[0], b1[1], b1[2], 0.0f);
   }
+  if (bad) atomicOr(err, bad);
   __shared__ float red[2][3][kBlock / 64];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   for (int a = 0; a < 3; a++) {
@@ -236,7 +237,8 @@ __global__ __launch_bounds__(kBlock) void k_range_counts(uint32_t ni, const uint
 __device__ inline float pad_lo(float x) { return x - fabsf(x) * 2.4e-7f - 1e-30f; }
 __device__ inline float pad_hi(float x) { return x + fabsf(x) * 2.4e-7f + 1e-30f; }
 
-// Step 6.
+// Step 6.  Grid-stride, so that the node count and depth take two atomics per block of at most
+// kWideBlocks (two per reachable node took most of its 0.78 ms).
 __global__ __launch_bounds__(kBlock) void k_layout(int n, const uint32_t* __restrict__ vals,
                                                    const float4* __restrict__ flo, const float4* __restrict__ fhi,
                                                    const uint32_t* __restrict__ child, const uint32_t* __restrict__ range,
@@ -245,48 +247,63 @@ __global__ __launch_bounds__(kBlock) void k_layout(int n, const uint32_t* __rest
                                                    const uint8_t* __restrict__ collapse, Node2* __restrict__ nodes,
                                                    uint32_t* stats /* [0]=reachable interior, [1]=max depth */,
                                                    uint8_t* __restrict__ reach) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n - 1) return;
-  float4 lo[2], hi[2];
-  int ref[2];
-  for (int c = 0; c < 2; c++) {
-    const uint32_t ch = child[2 * i + c];
-    if (ch & kLeafBit) {
-      const uint32_t k = ch & ~kLeafBit;
-      const uint32_t f = vals[k];
-      lo[c] = flo[f];
-      hi[c] = fhi[f];
-      ref[c] = make_leaf_ref(k, 1u);
-    } else {
-      lo[c] = node_lo[ch];
-      hi[c] = node_hi[ch];
-      if (collapse[ch]) {
-        const uint32_t first = range[2 * ch], last = range[2 * ch + 1];
-        ref[c] = make_leaf_ref(first, last - first + 1u);
+  uint32_t found = 0, deepest = 0;
+  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n - 1; i += gridDim.x * kBlock) {
+    float4 lo[2], hi[2];
+    int ref[2];
+    for (int c = 0; c < 2; c++) {
+      const uint32_t ch = child[2 * i + c];
+      if (ch & kLeafBit) {
+        const uint32_t k = ch & ~kLeafBit;
+        const uint32_t f = vals[k];
+        lo[c] = flo[f];
+        hi[c] = fhi[f];
+        ref[c] = make_leaf_ref(k, 1u);
       } else {
-        ref[c] = static_cast<int>(ch);
+        lo[c] = node_lo[ch];
+        hi[c] = node_hi[ch];
+        if (collapse[ch]) {
+          const uint32_t first = range[2 * ch], last = range[2 * ch + 1];
+          ref[c] = make_leaf_ref(first, last - first + 1u);
+        } else {
+          ref[c] = static_cast<int>(ch);
+        }
       }
     }
+    Node2 nd;
+    nd.a = make_float4(pad_lo(lo[0].x), pad_hi(hi[0].x), pad_lo(lo[0].y), pad_hi(hi[0].y));
+    nd.b = make_float4(pad_lo(lo[1].x), pad_hi(hi[1].x), pad_lo(lo[1].y), pad_hi(hi[1].y));
+    nd.c = make_float4(pad_lo(lo[0].z), pad_hi(hi[0].z), pad_lo(lo[1].z), pad_hi(hi[1].z));
+    nd.d = make_int4(ref[0], ref[1], 0, 0);
+    nodes[i] = nd;
+    // reachable iff neither this node nor an ancestor became a leaf
+    bool reachable = collapse[i] == 0;
+    uint32_t depth = 0;
+    int p = i;
+    while (reachable && p != 0) {
+      p = parent_int[p];
+      depth++;
+      if (collapse[p]) reachable = false;
+    }
+    reach[i] = reachable ? 1 : 0;
+    if (reachable) {
+      found++;
+      deepest = max(deepest, depth + 1u);
+    }
   }
-  Node2 nd;
-  nd.a = make_float4(pad_lo(lo[0].x), pad_hi(hi[0].x), pad_lo(lo[0].y), pad_hi(hi[0].y));
-  nd.b = make_float4(pad_lo(lo[1].x), pad_hi(hi[1].x), pad_lo(lo[1].y), pad_hi(hi[1].y));
-  nd.c = make_float4(pad_lo(lo[0].z), pad_hi(hi[0].z), pad_lo(lo[1].z), pad_hi(hi[1].z));
-  nd.d = make_int4(ref[0], ref[1], 0, 0);
-  nodes[i] = nd;
-  // reachable iff neither this node nor an ancestor became a leaf
-  bool reachable = collapse[i] == 0;
-  uint32_t depth = 0;
-  int p = i;
-  while (reachable && p != 0) {
-    p = parent_int[p];
-    depth++;
-    if (collapse[p]) reachable = false;
+  for (int off = 32; off > 0; off >>= 1) {
+    found += __shfl_xor(found, off, 64);
+    deepest = max(deepest, static_cast<uint32_t>(__shfl_xor(deepest, off, 64)));
   }
-  reach[i] = reachable ? 1 : 0;
-  if (reachable) {
-    atomicAdd(&stats[0], 1u);
-    atomicMax(&stats[1], depth + 1u);
+  __shared__ uint32_t red[2][kBlock / 64];
+  if ((threadIdx.x & 63) == 0) { red[0][threadIdx.x >> 6] = found; red[1][threadIdx.x >> 6] = deepest; }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kBlock / 64; w++) { found += red[0][w]; deepest = max(deepest, red[1][w]); }
+    if (found > 0) {
+      atomicAdd(&stats[0], found);
+      atomicMax(&stats[1], deepest);
+    }
   }
 }
 
@@ -398,54 +415,10 @@ __global__ __launch_bounds__(kBlock) void k_leaf_boxes(uint32_t nf, const uint32
   o[0] = a.x; o[1] = a.y; o[2] = a.z; o[3] = b.x; o[4] = b.y; o[5] = b.z;
 }
 
-// Treelet restructuring of `root` by one whole wave (all 64 lanes call it with the same
-// root): every lane forms the same treelet; the areas of the leaf subsets (two per lane)
-// and then, subset size by subset size, their optimal costs and splits are computed in
-// LDS (a subset's splits only use smaller subsets); lane 0 rebuilds the treelet.  The
-// per-subset choices are those of the serial treelet_optimize().
-__device__ void treelet_wave(const TreeArrays& t, int root, float c_node, float c_tri, float* s_area, float* s_copt,
-                             uint8_t* s_part) {
-  // the treelet (formed by lane 0) and its leaf boxes (one lane each) live in LDS: held per
-  // lane, the arrays were private memory that all 64 lanes wrote and read
-  __shared__ uint32_t s_leaf[kTreeletLeaves];
-  __shared__ int s_inner[kTreeletLeaves - 1];
-  __shared__ float s_lb[kTreeletLeaves][6];
-  __shared__ int s_nl;
-  const int lane = threadIdx.x;
-  if (lane == 0) s_nl = treelet_form(t, root, s_leaf, s_inner);
-  __syncthreads();
-  const int nl = s_nl;
-  if (nl < 3) return;  // the same for every lane
-  if (lane < nl) ref_box(t, s_leaf[lane], s_lb[lane]);
-  __syncthreads();
-  const uint32_t full = (1u << nl) - 1u;
-  for (uint32_t S = lane; S <= full; S += 64)
-    if (S >= 1) s_area[S] = subset_area(s_lb, nl, S);
-  if (lane < nl) {
-    s_copt[1u << lane] = ref_cost(t, s_leaf[lane], c_tri);
-    s_part[1u << lane] = 0;
-  }
-  __syncthreads();
-  for (int size = 2; size <= nl; size++) {
-    for (uint32_t S = lane; S <= full; S += 64) {
-      if (S >= 1 && popcount7(S) == size) {
-        uint32_t bp;
-        s_copt[S] = best_split(s_copt, S, s_area[S], c_node, &bp);
-        s_part[S] = static_cast<uint8_t>(bp);
-      }
-    }
-    __syncthreads();
-  }
-  const bool better = s_copt[full] < t.cost[root] * (1.0f - 1e-6f);
-  if (better && lane == 0) treelet_rebuild(t, root, s_leaf, s_inner, nl, s_part, c_node, c_tri);
-  __syncthreads();
-}
-
 // One bottom-up treelet pass runs level by level over the current tree, deepest first
 // (make_levels): at each depth, k_refresh_nodes sets the box, count and cost of the nodes
 // with fewer than `gamma` triangles below from their children (thread per node), and
-// k_treelet_nodes does the same for the others and restructures each with one wave
-// (treelet_wave).  Children are final when their parent's level runs (earlier launches), a
+// k_treelet_nodes does the same for the others and restructures each with one wave.  Children are final when their parent's level runs (earlier launches), a
 // treelet only involves nodes of its subtree, and the nodes of one depth have disjoint
 // subtrees, so no counters or fences are needed.  Which nodes get a treelet is known in
 // advance: a node's triangle count depends only on its leaf set, which restructuring below
@@ -456,15 +429,284 @@ __global__ __launch_bounds__(kBlock) void k_refresh_nodes(const uint32_t* __rest
   if (k < hi) refresh_node(t, static_cast<int>(order[k]), c_node, c_tri);
 }
 
+// One treelet leaf, held by one lane.
+struct TreeletLeaf {
+  uint32_t ref;
+  uint32_t ch0, ch1;  // children of an interior leaf
+  float b[6];
+  float area;         // half area of an interior leaf, -1 for a triangle: what to open next
+  float cost;
+  uint32_t count;
+};
+
+__device__ __forceinline__ float half_area_of(const float* b) {
+  const float dx = b[3] - b[0], dy = b[4] - b[1], dz = b[5] - b[2];
+  return dx * dy + dy * dz + dz * dx;
+}
+
+__device__ __forceinline__ void load_treelet_leaf(const TreeArrays& t, uint32_t ref, float c_tri, TreeletLeaf& l) {
+  const bool tri = (ref & kTreeLeafBit) != 0;
+  const uint32_t i = ref & ~kTreeLeafBit;
+  const float2* b = reinterpret_cast<const float2*>((tri ? t.leaf_box : t.box) + 6 * static_cast<size_t>(i));
+  uint2 ch = make_uint2(0u, 0u);
+  float cost = 0.0f;
+  uint32_t count = 1u;
+  if (!tri) {
+    ch = *reinterpret_cast<const uint2*>(t.child + 2 * static_cast<size_t>(i));
+    cost = t.cost[i];
+    count = t.count[i];
+  }
+  const float2 b0 = b[0], b1 = b[1], b2 = b[2];
+  l.ref = ref;
+  l.ch0 = ch.x;
+  l.ch1 = ch.y;
+  l.b[0] = b0.x; l.b[1] = b0.y; l.b[2] = b1.x; l.b[3] = b1.y; l.b[4] = b2.x; l.b[5] = b2.y;
+  const float area = half_area_of(l.b);
+  l.area = tri ? -1.0f : area;
+  l.cost = tri ? c_tri * area : cost;
+  l.count = count;
+}
+
+__device__ __forceinline__ uint32_t lane_u32(uint32_t v, uint32_t lane) { return __builtin_amdgcn_readlane(v, lane); }
+__device__ __forceinline__ float lane_f32(float v, uint32_t lane) {
+  return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane));
+}
+
+// The seven-leaf treelet below every node of order[lo, lo + grid), one wave each: box, count
+// and cost of the node from its children, then treelet_form, the dynamic program and
+// treelet_rebuild of rmh_treelet.hpp with the same choices and the same arithmetic (the trees
+// are those of the serial treelet_optimize()).  A node that gets a treelet has at least seven
+// triangles below it, so it always has seven leaves.
+//
+// What bounds it is the length of one treelet's chain, so nothing in it is serial that need
+// not be: lane j holds leaf j of the growing treelet with its box, cost and children, so
+// opening a leaf is one dependent load round; the 127 subset areas take two subsets per lane
+// (S and S + 64, whose boxes differ by leaf 6); subsets of up to five leaves have their splits
+// walked by one lane each (at most 15), the 7 subsets of six are shared by 8 lanes each (4
+// splits per lane) and the 63 splits of the whole treelet by all lanes; the new topology is
+// built in registers and its six nodes are written by six lanes.  With the treelet formed and
+// rebuilt by lane 0 through memory, and every subset's splits walked by one lane (126 steps
+// for the whole treelet), three rounds on the 2.1M-triangle terrain took 11.2 ms, 3.1 ms now.
 __global__ __launch_bounds__(64) void k_treelet_nodes(const uint32_t* __restrict__ order, uint32_t lo, TreeArrays t,
                                                       float c_node, float c_tri) {
-  __shared__ float s_area[1 << kTreeletLeaves];
-  __shared__ float s_copt[1 << kTreeletLeaves];
-  __shared__ uint8_t s_part[1 << kTreeletLeaves];
-  const int p = static_cast<int>(order[lo + blockIdx.x]);
-  if (threadIdx.x == 0) refresh_node(t, p, c_node, c_tri);
-  __syncthreads();  // lane 0's box and cost before the wave reads them
-  treelet_wave(t, p, c_node, c_tri, s_area, s_copt, s_part);
+  static_assert(kTreeletLeaves == 7, "lanes are laid out for seven leaves");
+  __shared__ float s_copt[128];
+  __shared__ uint8_t s_part[128];
+  const uint32_t lane = threadIdx.x;
+  const uint32_t root = __builtin_amdgcn_readfirstlane(order[lo + blockIdx.x]);
+
+  // the treelet: lanes 0 and 1 start with the root's children; the interior leaf of largest
+  // area (the first of equals) is opened, its children go to its lane and to the next one
+  TreeletLeaf leaf;
+  leaf.area = -1.0f;
+  const uint2 rc = *reinterpret_cast<const uint2*>(t.child + 2 * static_cast<size_t>(root));
+  if (lane < 2) load_treelet_leaf(t, lane == 0 ? rc.x : rc.y, c_tri, leaf);
+  float root_box[6];
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    const float a0 = lane_f32(leaf.b[k], 0), a1 = lane_f32(leaf.b[k], 1);
+    const float h0 = lane_f32(leaf.b[3 + k], 0), h1 = lane_f32(leaf.b[3 + k], 1);
+    root_box[k] = a0 < a1 ? a0 : a1;
+    root_box[3 + k] = h0 > h1 ? h0 : h1;
+  }
+  const float root_cost = c_node * half_area_of(root_box) + lane_f32(leaf.cost, 0) + lane_f32(leaf.cost, 1);
+  const uint32_t root_count = lane_u32(leaf.count, 0) + lane_u32(leaf.count, 1);
+  uint32_t inner = root;  // lane i: the i-th interior node of the treelet
+#pragma unroll
+  for (uint32_t nl = 2; nl < 7; nl++) {
+    float a = leaf.area;
+    uint32_t best = lane;
+#pragma unroll
+    for (int off = 4; off > 0; off >>= 1) {
+      const float oa = __shfl_xor(a, off, 8);
+      const uint32_t ob = __shfl_xor(best, off, 8);
+      const bool take = oa > a || (oa == a && ob < best);
+      a = take ? oa : a;
+      best = take ? ob : best;
+    }
+    best = __builtin_amdgcn_readfirstlane(best);
+    const uint32_t x = lane_u32(leaf.ref, best), c0 = lane_u32(leaf.ch0, best), c1 = lane_u32(leaf.ch1, best);
+    if (lane == nl - 1) inner = x;
+    if (lane == best || lane == nl) load_treelet_leaf(t, lane == best ? c0 : c1, c_tri, leaf);
+  }
+
+  // areas of the subsets lane (leaves 0-5) and lane + 64 (with leaf 6)
+  float bx[6] = {3.0e38f, 3.0e38f, 3.0e38f, -3.0e38f, -3.0e38f, -3.0e38f};
+#pragma unroll
+  for (uint32_t j = 0; j < 6; j++) {
+    const bool in = (lane >> j) & 1u;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      const float l = lane_f32(leaf.b[k], j), h = lane_f32(leaf.b[3 + k], j);
+      bx[k] = in && l < bx[k] ? l : bx[k];
+      bx[3 + k] = in && h > bx[3 + k] ? h : bx[3 + k];
+    }
+  }
+  const float area_lo = half_area_of(bx);
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    const float l = lane_f32(leaf.b[k], 6), h = lane_f32(leaf.b[3 + k], 6);
+    bx[k] = l < bx[k] ? l : bx[k];
+    bx[3 + k] = h > bx[3 + k] ? h : bx[3 + k];
+  }
+  const float area_hi = half_area_of(bx);
+
+  // least costs and splits, subset size by subset size: a split is the part P that holds the
+  // lowest member, P's other members a proper subset r of the rest, in descending order, the
+  // first of equals kept
+  if (lane < 7) s_copt[1u << lane] = leaf.cost;
+  __syncthreads();
+  const uint32_t members = __popc(lane);
+#pragma unroll
+  for (uint32_t size = 2; size <= 5; size++) {
+    const bool high = members == size - 1;
+    if (high || members == size) {
+      const uint32_t S = high ? lane + 64u : lane;
+      const uint32_t low = S & (0u - S), rest = S ^ low;
+      float best = 3.0e38f;
+      uint32_t bp = low;
+      uint32_t r = rest;
+#pragma unroll
+      for (uint32_t k = 0; k < (1u << (size - 1)) - 1u; k++) {
+        r = (r - 1u) & rest;
+        const float c = s_copt[low | r] + s_copt[rest ^ r];
+        if (c < best) { best = c; bp = low | r; }
+      }
+      s_copt[S] = c_node * (high ? area_hi : area_lo) + best;
+      s_part[S] = static_cast<uint8_t>(bp);
+    }
+    __syncthreads();
+  }
+  {
+    // six leaves: subset 127 without leaf m, 8 lanes each; split j (of 31) in the compressed
+    // index of its five other members, the larger of equals
+    const uint32_t m = lane >> 3, S = 127u ^ (1u << m);
+    float best = 3.0e38f;
+    uint32_t bj = 0;
+    if (m < 7) {
+#pragma unroll
+      for (uint32_t q = 0; q < 4; q++) {
+        const uint32_t j = (lane & 7u) + 8u * q;
+        if (j < 31u) {
+          const uint32_t x = 1u | (j << 1);
+          const uint32_t P = ((x >> m) << (m + 1)) | (x & ((1u << m) - 1u));
+          const float c = s_copt[P] + s_copt[S ^ P];
+          if (c <= best) { best = c; bj = j; }
+        }
+      }
+    }
+#pragma unroll
+    for (int off = 4; off > 0; off >>= 1) {
+      const float oc = __shfl_xor(best, off, 8);
+      const uint32_t oj = __shfl_xor(bj, off, 8);
+      const bool take = oc < best || (oc == best && oj > bj);
+      best = take ? oc : best;
+      bj = take ? oj : bj;
+    }
+    const float area_m = __shfl(area_hi, static_cast<int>(63u ^ (1u << m)) & 63, 64);  // by all lanes
+    const float area = m == 6 ? lane_f32(area_lo, 63) : area_m;
+    if (m < 7 && (lane & 7u) == 0) {
+      const uint32_t x = 1u | (bj << 1);
+      s_copt[S] = c_node * area + best;
+      s_part[S] = static_cast<uint8_t>(((x >> m) << (m + 1)) | (x & ((1u << m) - 1u)));
+    }
+  }
+  __syncthreads();
+  float best = 3.0e38f;
+  uint32_t bj = 0;
+  if (lane < 63) {
+    const uint32_t P = 1u | (lane << 1);
+    const float c = s_copt[P] + s_copt[127u ^ P];
+    if (c < best) { best = c; bj = lane; }
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const float oc = __shfl_xor(best, off, 64);
+    const uint32_t oj = __shfl_xor(bj, off, 64);
+    const bool take = oc < best || (oc == best && oj > bj);
+    best = take ? oc : best;
+    bj = take ? oj : bj;
+  }
+  best = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(best)));
+  const uint32_t part_all = 1u | (__builtin_amdgcn_readfirstlane(bj) << 1);
+  const float copt_all = c_node * lane_f32(area_hi, 63) + best;
+  if (!(copt_all < root_cost * (1.0f - 1e-6f))) {
+    // the topology stays: the node's own box, count and cost
+    if (lane == 0) {
+#pragma unroll
+      for (int k = 0; k < 6; k++) t.box[6 * static_cast<size_t>(root) + k] = root_box[k];
+      t.count[root] = root_count;
+      t.cost[root] = root_cost;
+    }
+    return;
+  }
+
+  // the new topology, built by all lanes alike: slot i (lane i) is the i-th interior node;
+  // subsets still to be split wait on a stack (lane = position)
+  uint32_t st_set = 127u, st_slot = 0u;                       // the stack
+  uint32_t n_set = 0u, n_ref0 = 0u, n_ref1 = 0u;              // lane i: slot i
+  uint32_t n_c0 = 0u, n_c1 = 0u;                              // its children: leaf j, or 8 + slot
+  uint32_t made = 0u;                                         // slots in the order they were made, 4 bits each
+  uint32_t sp = 1u, next = 1u;
+#pragma unroll
+  for (uint32_t k = 0; k < 6; k++) {
+    sp--;
+    const uint32_t S = lane_u32(st_set, sp), slot = lane_u32(st_slot, sp);
+    made |= slot << (4 * k);
+    const uint32_t P = S == 127u ? part_all : __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(s_part[S]));
+    uint32_t refs[2], kids[2];
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      const uint32_t sub = c ? S ^ P : P;
+      if ((sub & (sub - 1u)) == 0u) {
+        kids[c] = __builtin_ctz(sub);
+        refs[c] = lane_u32(leaf.ref, kids[c]);
+      } else {
+        kids[c] = 8u + next;
+        refs[c] = lane_u32(inner, next);
+        if (lane == sp) { st_set = sub; st_slot = next; }
+        sp++;
+        next++;
+      }
+    }
+    if (lane == slot) { n_set = S; n_ref0 = refs[0]; n_ref1 = refs[1]; n_c0 = kids[0]; n_c1 = kids[1]; }
+  }
+  // costs bottom-up in reverse order of making
+  float n_cost = 0.0f;
+#pragma unroll
+  for (int k = 5; k >= 0; k--) {
+    const uint32_t slot = (made >> (4 * k)) & 15u;
+    const uint32_t S = lane_u32(n_set, slot), k0 = lane_u32(n_c0, slot), k1 = lane_u32(n_c1, slot);
+    const float area = S >= 64u ? lane_f32(area_hi, S - 64u) : lane_f32(area_lo, S);
+    const float cost0 = k0 < 8u ? lane_f32(leaf.cost, k0) : lane_f32(n_cost, k0 - 8u);
+    const float cost1 = k1 < 8u ? lane_f32(leaf.cost, k1) : lane_f32(n_cost, k1 - 8u);
+    const float cost = c_node * area + cost0 + cost1;
+    if (lane == slot) n_cost = cost;
+  }
+  float nb[6] = {3.0e38f, 3.0e38f, 3.0e38f, -3.0e38f, -3.0e38f, -3.0e38f};
+  uint32_t n_count = 0u;
+#pragma unroll
+  for (uint32_t j = 0; j < 7; j++) {
+    const bool in = (n_set >> j) & 1u;
+    n_count += in ? lane_u32(leaf.count, j) : 0u;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      const float l = lane_f32(leaf.b[k], j), h = lane_f32(leaf.b[3 + k], j);
+      nb[k] = in && l < nb[k] ? l : nb[k];
+      nb[3 + k] = in && h > nb[3 + k] ? h : nb[3 + k];
+    }
+  }
+  if (lane < 6) {
+    *reinterpret_cast<uint2*>(t.child + 2 * static_cast<size_t>(inner)) = make_uint2(n_ref0, n_ref1);
+    float2* b = reinterpret_cast<float2*>(t.box + 6 * static_cast<size_t>(inner));
+    b[0] = make_float2(nb[0], nb[1]);
+    b[1] = make_float2(nb[2], nb[3]);
+    b[2] = make_float2(nb[4], nb[5]);
+    t.count[inner] = n_count;
+    t.cost[inner] = n_cost;
+    set_parent(t, n_ref0, static_cast<int>(inner));
+    set_parent(t, n_ref1, static_cast<int>(inner));
+  }
 }
 
 // Structure check of the refined tree before anything walks it: every child slot points
@@ -1007,7 +1249,7 @@ static int map_build(const float* vertices, uint32_t nv, const uint32_t* faces, 
 
   BUILD_TRY(hipEventRecord(ev0, stream));
   k_init<<<1, 64, 0, stream>>>(bounds.as<float>(), err.as<uint32_t>());
-  k_prep<<<blocks_for(nf), kBlock, 0, stream>>>(m->vertices, nv, m->faces, nf, flo.as<float4>(), fhi.as<float4>(),
+  k_prep<<<std::min(blocks_for(nf), kWideBlocks), kBlock, 0, stream>>>(m->vertices, nv, m->faces, nf, flo.as<float4>(), fhi.as<float4>(),
                                                 bounds.as<float>(), err.as<uint32_t>());
   BUILD_TRY(hipGetLastError());
   uint32_t herr = 0;
@@ -1106,7 +1348,7 @@ static int map_build(const float* vertices, uint32_t nv, const uint32_t* faces, 
                                                                 prm.sah_cost_node, prm.sah_cost_tri);
       BUILD_TRY(hipGetLastError());
     }
-    k_layout<<<blocks_for(ni), kBlock, 0, stream>>>(n, svals, flo.as<float4>(), fhi.as<float4>(), child.as<uint32_t>(),
+    k_layout<<<std::min(blocks_for(ni), kWideBlocks), kBlock, 0, stream>>>(n, svals, flo.as<float4>(), fhi.as<float4>(), child.as<uint32_t>(),
                                                     range.as<uint32_t>(), pint.as<int>(), nlo.as<float4>(),
                                                     nhi.as<float4>(), coll.as<uint8_t>(), m->nodes, stats.as<uint32_t>(),
                                                     m->reach);
