@@ -926,6 +926,43 @@ __global__ __launch_bounds__(kBlock) void k_wide_emit(const Node2* __restrict__ 
   out[base + j] = nd;
 }
 
+// Arrays laid out one after another in one block, 256-byte aligned: with base NULL only the
+// size is counted.
+struct Carve {
+  char* base = nullptr;
+  size_t size = 0;
+  template <class T>
+  T* take(size_t n) {
+    T* p = reinterpret_cast<T*>(base ? base + size : nullptr);
+    size += (n * sizeof(T) + 255) & ~static_cast<size_t>(255);
+    return p;
+  }
+};
+
+// One block of scratch from the library's pool (from hipMalloc when the pool cannot give it),
+// handed back in stream order.
+struct Scratch {
+  void* p = nullptr;
+  bool pooled = false;
+  hipStream_t stream = nullptr;
+  hipError_t alloc(int device, size_t bytes, hipStream_t s) {
+    stream = s;
+    const hipMemPool_t pool = scratch_pool(device);
+    if (pool && hipMallocFromPoolAsync(&p, bytes, pool, s) == hipSuccess) {
+      pooled = true;
+      return hipSuccess;
+    }
+    (void)hipGetLastError();
+    p = nullptr;
+    return hipMalloc(&p, bytes);
+  }
+  ~Scratch() {
+    if (!p) return;
+    if (pooled) (void)hipFreeAsync(p, stream);
+    else (void)hipFree(p);
+  }
+};
+
 struct DevBuf {
   void* p = nullptr;
   ~DevBuf() { if (p) (void)hipFree(p); }
@@ -941,26 +978,26 @@ struct LevelClass {
   bool treelet;
 };
 
-// Scratch of make_levels for a tree of ni interior nodes.
-struct LevelBufs {
-  DevBuf keys, keys2, idx, order, start, tmp;
-  size_t tmp_bytes = 0;
-};
-
 constexpr uint32_t kLevelKeys = 2u * (static_cast<uint32_t>(kMaxTreeWalk) + 1u);
 
-hipError_t level_bufs(LevelBufs& b, uint32_t ni, hipStream_t stream) {
-  hipError_t e;
-  if ((e = hipMalloc(&b.keys.p, sizeof(uint32_t) * ni)) != hipSuccess) return e;
-  if ((e = hipMalloc(&b.keys2.p, sizeof(uint32_t) * ni)) != hipSuccess) return e;
-  if ((e = hipMalloc(&b.idx.p, sizeof(uint32_t) * ni)) != hipSuccess) return e;
-  if ((e = hipMalloc(&b.order.p, sizeof(uint32_t) * ni)) != hipSuccess) return e;
-  if ((e = hipMalloc(&b.start.p, sizeof(uint32_t) * kLevelKeys)) != hipSuccess) return e;
-  e = rocprim::radix_sort_pairs(nullptr, b.tmp_bytes, b.keys.as<uint32_t>(), b.keys2.as<uint32_t>(),
-                                b.idx.as<uint32_t>(), b.order.as<uint32_t>(), ni, 0u, 14u, stream);
-  if (e != hipSuccess) return e;
-  return hipMalloc(&b.tmp.p, b.tmp_bytes);
-}
+// Scratch of make_levels for a tree of ni interior nodes.
+struct LevelBufs {
+  uint32_t *keys = nullptr, *keys2 = nullptr, *idx = nullptr, *order = nullptr, *start = nullptr;
+  char* tmp = nullptr;
+  size_t tmp_bytes = 0;
+
+  hipError_t sort(uint32_t ni, hipStream_t stream) {
+    return rocprim::radix_sort_pairs(tmp, tmp_bytes, keys, keys2, idx, order, ni, 0u, 14u, stream);
+  }
+  void carve(Carve& c, uint32_t ni) {
+    keys = c.take<uint32_t>(ni);
+    keys2 = c.take<uint32_t>(ni);
+    idx = c.take<uint32_t>(ni);
+    order = c.take<uint32_t>(ni);
+    start = c.take<uint32_t>(kLevelKeys);
+    tmp = c.take<char>(tmp_bytes);
+  }
+};
 
 // Interior nodes of the radix tree (n leaves, n - 1 interior nodes) grouped by depth,
 // deepest first, into b.order; `classes` receives the launch ranges in that order (within a
@@ -970,17 +1007,15 @@ hipError_t make_levels(int n, const int* parent_int, const uint32_t* count, uint
                        uint32_t* err, hipStream_t stream, std::vector<LevelClass>& classes) {
   const uint32_t ni = static_cast<uint32_t>(n - 1);
   hipError_t e;
-  k_level_keys<<<blocks_for(ni), kBlock, 0, stream>>>(n, parent_int, count, gamma, b.keys.as<uint32_t>(),
-                                                      b.idx.as<uint32_t>(), err);
+  k_level_keys<<<blocks_for(ni), kBlock, 0, stream>>>(n, parent_int, count, gamma, b.keys,
+                                                      b.idx, err);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  if ((e = rocprim::radix_sort_pairs(b.tmp.p, b.tmp_bytes, b.keys.as<uint32_t>(), b.keys2.as<uint32_t>(),
-                                     b.idx.as<uint32_t>(), b.order.as<uint32_t>(), ni, 0u, 14u, stream)) != hipSuccess)
-    return e;
-  if ((e = hipMemsetAsync(b.start.p, 0xFF, sizeof(uint32_t) * kLevelKeys, stream)) != hipSuccess) return e;
-  k_level_starts<<<blocks_for(ni), kBlock, 0, stream>>>(ni, b.keys2.as<uint32_t>(), b.start.as<uint32_t>());
+  if ((e = b.sort(ni, stream)) != hipSuccess) return e;
+  if ((e = hipMemsetAsync(b.start, 0xFF, sizeof(uint32_t) * kLevelKeys, stream)) != hipSuccess) return e;
+  k_level_starts<<<blocks_for(ni), kBlock, 0, stream>>>(ni, b.keys2, b.start);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   std::vector<uint32_t> st(kLevelKeys);
-  if ((e = hipMemcpyAsync(st.data(), b.start.p, sizeof(uint32_t) * kLevelKeys, hipMemcpyDeviceToHost, stream)) !=
+  if ((e = hipMemcpyAsync(st.data(), b.start, sizeof(uint32_t) * kLevelKeys, hipMemcpyDeviceToHost, stream)) !=
       hipSuccess)
     return e;
   if ((e = hipStreamSynchronize(stream)) != hipSuccess) return e;
@@ -995,13 +1030,8 @@ hipError_t make_levels(int n, const int* parent_int, const uint32_t* count, uint
 
 void map_free(rmh_map* m) {
   if (!m) return;
-  if (m->vertices) (void)hipFree(m->vertices);
-  if (m->faces) (void)hipFree(m->faces);
-  if (m->tris) (void)hipFree(m->tris);
-  if (m->normals) (void)hipFree(m->normals);
-  if (m->nodes) (void)hipFree(m->nodes);
-  if (m->parent) (void)hipFree(m->parent);
-  if (m->reach) (void)hipFree(m->reach);
+  if (m->mesh_block) (void)hipFree(m->mesh_block);
+  if (m->tree_block) (void)hipFree(m->tree_block);
   if (m->nodes4) (void)hipFree(m->nodes4);
   if (m->refit_order) (void)hipFree(m->refit_order);
   delete m;
@@ -1091,50 +1121,42 @@ hipError_t build_wide(rmh_map* m, hipStream_t stream) {
 
 }  // namespace
 
-// Rewrites m->nodes / m->parent / m->reach (ni radix-tree slots, n_reach of them reachable,
-// root at slot 0, size = interior nodes of the final tree per subtree) into preorder, in
-// buffers of exactly n_reach entries.
-static hipError_t preorder_nodes(rmh_map* m, uint32_t ni, uint32_t n_reach, const uint32_t* size,
+// Writes the n_reach reachable nodes of the ni radix-tree slots (root at slot 0; size =
+// interior nodes of the final tree per subtree), their parents and reach flags in preorder
+// into the map's tree block.  rank and err are scratch.
+static hipError_t preorder_nodes(rmh_map* m, uint32_t ni, uint32_t n_reach, const Node2* nodes, const int* parent,
+                                 const uint8_t* reach, const uint32_t* size, uint32_t* rank, uint32_t* err,
                                  hipStream_t stream) {
-  DevBuf rank, err;
-  Node2* nodes = nullptr;
-  int* parent = nullptr;
-  uint8_t* reach = nullptr;
-  hipError_t e = hipMalloc(&rank.p, sizeof(uint32_t) * ni);
-  if (e == hipSuccess) e = hipMalloc(&err.p, sizeof(uint32_t));
-  if (e == hipSuccess) e = hipMalloc(&nodes, sizeof(Node2) * n_reach);
-  if (e == hipSuccess) e = hipMalloc(&parent, sizeof(int) * n_reach);
-  if (e == hipSuccess) e = hipMalloc(&reach, n_reach);
-  if (e == hipSuccess) e = hipMemsetAsync(err.p, 0, sizeof(uint32_t), stream);
+  Carve c;
+  for (int pass = 0; pass < 2; pass++) {
+    c.size = 0;
+    m->nodes = c.take<Node2>(n_reach);
+    m->parent = c.take<int>(n_reach);
+    m->reach = c.take<uint8_t>(n_reach);
+    if (pass == 0) {
+      const hipError_t e = hipMalloc(&m->tree_block, c.size);
+      if (e != hipSuccess) { m->tree_block = nullptr; return e; }
+      c.base = static_cast<char*>(m->tree_block);
+    }
+  }
+  hipError_t e = hipMemsetAsync(err, 0, sizeof(uint32_t), stream);
   if (e == hipSuccess) {
-    k_preorder_rank<<<blocks_for(ni), kBlock, 0, stream>>>(ni, m->reach, m->parent, m->nodes, size,
-                                                           rank.as<uint32_t>(), err.as<uint32_t>());
+    k_preorder_rank<<<blocks_for(ni), kBlock, 0, stream>>>(ni, reach, parent, nodes, size, rank, err);
     e = hipGetLastError();
   }
   if (e == hipSuccess) {
-    k_preorder_scatter<<<blocks_for(ni), kBlock, 0, stream>>>(ni, n_reach, m->reach, m->parent, m->nodes,
-                                                              rank.as<uint32_t>(), nodes, parent, reach, err.as<uint32_t>());
+    k_preorder_scatter<<<blocks_for(ni), kBlock, 0, stream>>>(ni, n_reach, reach, parent, nodes, rank, m->nodes,
+                                                              m->parent, m->reach, err);
     e = hipGetLastError();
   }
   uint32_t herr = 0, root_size = 0;
-  if (e == hipSuccess) e = hipMemcpyAsync(&herr, err.p, sizeof(uint32_t), hipMemcpyDeviceToHost, stream);
+  if (e == hipSuccess) e = hipMemcpyAsync(&herr, err, sizeof(uint32_t), hipMemcpyDeviceToHost, stream);
   if (e == hipSuccess) e = hipMemcpyAsync(&root_size, size, sizeof(uint32_t), hipMemcpyDeviceToHost, stream);
   if (e == hipSuccess) e = hipStreamSynchronize(stream);
   // a walk that did not end at the root, or a count that differs from the reachable
   // nodes, means the links do not form one tree: the build fails
   if (e == hipSuccess && (herr != 0 || root_size != n_reach)) e = hipErrorInvalidValue;
-  if (e != hipSuccess) {
-    if (nodes) (void)hipFree(nodes);
-    if (parent) (void)hipFree(parent);
-    if (reach) (void)hipFree(reach);
-    return e;
-  }
-  (void)hipFree(m->nodes);
-  (void)hipFree(m->parent);
-  (void)hipFree(m->reach);
-  m->nodes = nodes;
-  m->parent = parent;
-  m->reach = reach;
+  if (e != hipSuccess) return e;
   m->n_internal = n_reach;
   return hipSuccess;
 }
@@ -1210,152 +1232,179 @@ static int map_build(const float* vertices, uint32_t nv, const uint32_t* faces, 
   BUILD_TRY(hipEventCreate(&ev1));
   struct EvGuard { hipEvent_t a, b; ~EvGuard() { (void)hipEventDestroy(a); (void)hipEventDestroy(b); } } evg{ev0, ev1};
 
-  BUILD_TRY(hipMalloc(&m->vertices, sizeof(float) * 3 * nv));
-  BUILD_TRY(hipMalloc(&m->faces, sizeof(uint32_t) * 3 * nf));
+  Carve mc;
+  for (int pass = 0; pass < 2; pass++) {
+    mc.size = 0;
+    m->vertices = mc.take<float>(3 * static_cast<size_t>(nv));
+    m->faces = mc.take<uint32_t>(3 * static_cast<size_t>(nf));
+    m->tris = mc.take<float4>(3 * static_cast<size_t>(nf));
+    m->normals = mc.take<float4>(nf);
+    if (pass == 0) {
+      BUILD_TRY(hipMalloc(&m->mesh_block, mc.size));
+      mc.base = static_cast<char*>(m->mesh_block);
+    }
+  }
   BUILD_TRY(hipMemcpyAsync(m->vertices, vertices, sizeof(float) * 3 * nv, hipMemcpyDeviceToDevice, stream));
   BUILD_TRY(hipMemcpyAsync(m->faces, faces, sizeof(uint32_t) * 3 * nf, hipMemcpyDeviceToDevice, stream));
 
+  // All scratch is one block of the pool: 32 arrays allocated and freed one by one took 7 of
+  // the 14.5 ms of a 2.1M-triangle build.
   const int n = static_cast<int>(nf);
   const uint32_t ni = nf > 1 ? nf - 1 : 0;
-  DevBuf flo, fhi, bounds, err, keys, keys2, vals, vals2, child, range, pint, pleaf, nlo, nhi, coll, stats, moff, tmp,
-      subtree;
+  const bool refine = !(prm.flags & RMH_BVH_NO_REFINE) && n >= kTreeletLeaves;
+  float4 *flo, *fhi, *nlo, *nhi;
+  float *bounds, *lbox = nullptr, *tbox = nullptr, *tcost = nullptr;
+  uint32_t *err, *vals, *vals2, *child, *range, *stats, *moff, *subtree, *rank;
+  uint32_t *tcount = nullptr, *pos = nullptr, *offs = nullptr, *vals3 = nullptr, *refs = nullptr;
+  uint64_t *keys, *keys2;
+  int *pint, *pleaf, *pleaf2 = nullptr;
+  uint8_t *coll, *reach;
+  Node2* slots;  // nodes in radix-tree order
+  char* sort_tmp;
+  size_t sort_bytes = 0;
   LevelBufs lb;                    // scratch of the level-by-level passes (make_levels)
   std::vector<LevelClass> levels;  // their launch ranges
-  BUILD_TRY(hipMalloc(&flo.p, sizeof(float4) * nf));
-  BUILD_TRY(hipMalloc(&fhi.p, sizeof(float4) * nf));
-  BUILD_TRY(hipMalloc(&bounds.p, sizeof(float) * 8));
-  BUILD_TRY(hipMalloc(&err.p, sizeof(uint32_t) * 4));
-  BUILD_TRY(hipMalloc(&keys.p, sizeof(uint64_t) * nf));
-  BUILD_TRY(hipMalloc(&keys2.p, sizeof(uint64_t) * nf));
-  BUILD_TRY(hipMalloc(&vals.p, sizeof(uint32_t) * nf));
-  BUILD_TRY(hipMalloc(&vals2.p, sizeof(uint32_t) * nf));
-  BUILD_TRY(hipMalloc(&child.p, sizeof(uint32_t) * 2 * (ni + 1)));
-  BUILD_TRY(hipMalloc(&range.p, sizeof(uint32_t) * 2 * (ni + 1)));
-  BUILD_TRY(hipMalloc(&pint.p, sizeof(int) * (ni + 1)));
-  BUILD_TRY(hipMalloc(&pleaf.p, sizeof(int) * nf));
-  BUILD_TRY(hipMalloc(&nlo.p, sizeof(float4) * (ni + 1)));
-  BUILD_TRY(hipMalloc(&nhi.p, sizeof(float4) * (ni + 1)));
-  BUILD_TRY(hipMalloc(&coll.p, sizeof(uint8_t) * (ni + 1)));
-  BUILD_TRY(hipMalloc(&subtree.p, sizeof(uint32_t) * (ni + 1)));
-  if (ni > 0) BUILD_TRY(level_bufs(lb, ni, stream));
-  BUILD_TRY(hipMalloc(&stats.p, sizeof(uint32_t) * 4));
-  BUILD_TRY(hipMalloc(&moff.p, sizeof(uint32_t) * (n_meshes + 1)));
-  BUILD_TRY(hipMalloc(&m->tris, sizeof(float4) * 3 * static_cast<size_t>(nf)));
-  BUILD_TRY(hipMalloc(&m->normals, sizeof(float4) * nf));
-  BUILD_TRY(hipMalloc(&m->nodes, sizeof(Node2) * (ni + 1)));
-  BUILD_TRY(hipMalloc(&m->parent, sizeof(int) * (ni + 1)));
-  BUILD_TRY(hipMalloc(&m->reach, sizeof(uint8_t) * (ni + 1)));
-  BUILD_TRY(hipMemcpy(moff.p, off.data(), sizeof(uint32_t) * (n_meshes + 1), hipMemcpyHostToDevice));
+  BUILD_TRY(rocprim::radix_sort_pairs(nullptr, sort_bytes, static_cast<uint64_t*>(nullptr), static_cast<uint64_t*>(nullptr),
+                                      static_cast<uint32_t*>(nullptr), static_cast<uint32_t*>(nullptr), nf, 0u, 63u, stream));
+  if (ni > 0) BUILD_TRY(lb.sort(ni, stream));  // with tmp NULL: the size of its scratch
+  Scratch scratch;
+  Carve sc;
+  for (int pass = 0; pass < 2; pass++) {
+    sc.size = 0;
+    flo = sc.take<float4>(nf);
+    fhi = sc.take<float4>(nf);
+    bounds = sc.take<float>(8);
+    err = sc.take<uint32_t>(4);
+    stats = sc.take<uint32_t>(4);
+    moff = sc.take<uint32_t>(n_meshes + 1);
+    keys = sc.take<uint64_t>(nf);
+    keys2 = sc.take<uint64_t>(nf);
+    vals = sc.take<uint32_t>(nf);
+    vals2 = sc.take<uint32_t>(nf);
+    sort_tmp = sc.take<char>(sort_bytes);
+    child = sc.take<uint32_t>(2 * static_cast<size_t>(ni + 1));
+    range = sc.take<uint32_t>(2 * static_cast<size_t>(ni + 1));
+    pint = sc.take<int>(ni + 1);
+    pleaf = sc.take<int>(nf);
+    nlo = sc.take<float4>(ni + 1);
+    nhi = sc.take<float4>(ni + 1);
+    coll = sc.take<uint8_t>(ni + 1);
+    subtree = sc.take<uint32_t>(ni + 1);
+    slots = sc.take<Node2>(ni + 1);
+    reach = sc.take<uint8_t>(ni + 1);
+    rank = sc.take<uint32_t>(ni + 1);
+    if (ni > 0) lb.carve(sc, ni);
+    if (refine) {
+      lbox = sc.take<float>(6 * static_cast<size_t>(nf));
+      tbox = sc.take<float>(6 * static_cast<size_t>(ni));
+      tcost = sc.take<float>(ni);
+      tcount = sc.take<uint32_t>(ni);
+      pos = sc.take<uint32_t>(nf);
+      offs = sc.take<uint32_t>(ni);
+      vals3 = sc.take<uint32_t>(nf);
+      pleaf2 = sc.take<int>(nf);
+      refs = sc.take<uint32_t>(2 * static_cast<size_t>(nf) - 1);
+    }
+    if (pass == 0) {
+      BUILD_TRY(scratch.alloc(m->device, sc.size, stream));
+      sc.base = static_cast<char*>(scratch.p);
+    }
+  }
+  BUILD_TRY(hipMemcpyAsync(moff, off.data(), sizeof(uint32_t) * (n_meshes + 1), hipMemcpyHostToDevice, stream));
 
   BUILD_TRY(hipEventRecord(ev0, stream));
-  k_init<<<1, 64, 0, stream>>>(bounds.as<float>(), err.as<uint32_t>());
-  k_prep<<<std::min(blocks_for(nf), kWideBlocks), kBlock, 0, stream>>>(m->vertices, nv, m->faces, nf, flo.as<float4>(), fhi.as<float4>(),
-                                                bounds.as<float>(), err.as<uint32_t>());
+  k_init<<<1, 64, 0, stream>>>(bounds, err);
+  k_prep<<<std::min(blocks_for(nf), kWideBlocks), kBlock, 0, stream>>>(m->vertices, nv, m->faces, nf, flo, fhi,
+                                                bounds, err);
   BUILD_TRY(hipGetLastError());
   uint32_t herr = 0;
-  BUILD_TRY(hipMemcpyAsync(&herr, err.p, sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
+  BUILD_TRY(hipMemcpyAsync(&herr, err, sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
   BUILD_TRY(hipStreamSynchronize(stream));
   if (herr & 1u) { map_free(m); return fail(RMH_ERR_INVALID, "rmh_map_build: face index >= n_vertices"); }
   if (herr & 2u) { map_free(m); return fail(RMH_ERR_INVALID, "rmh_map_build: non-finite vertex coordinate"); }
 
-  k_morton<<<blocks_for(nf), kBlock, 0, stream>>>(flo.as<float4>(), fhi.as<float4>(), nf, bounds.as<float>(),
-                                                  keys.as<uint64_t>(), vals.as<uint32_t>());
+  k_morton<<<blocks_for(nf), kBlock, 0, stream>>>(flo, fhi, nf, bounds,
+                                                  keys, vals);
   BUILD_TRY(hipGetLastError());
-  size_t tmp_bytes = 0;
-  BUILD_TRY(rocprim::radix_sort_pairs(nullptr, tmp_bytes, keys.as<uint64_t>(), keys2.as<uint64_t>(),
-                                      vals.as<uint32_t>(), vals2.as<uint32_t>(), nf, 0u, 63u, stream));
-  BUILD_TRY(hipMalloc(&tmp.p, tmp_bytes));
-  BUILD_TRY(rocprim::radix_sort_pairs(tmp.p, tmp_bytes, keys.as<uint64_t>(), keys2.as<uint64_t>(),
-                                      vals.as<uint32_t>(), vals2.as<uint32_t>(), nf, 0u, 63u, stream));
-  uint64_t* skeys = keys2.as<uint64_t>();
-  uint32_t* svals = vals2.as<uint32_t>();
+  BUILD_TRY(rocprim::radix_sort_pairs(sort_tmp, sort_bytes, keys, keys2,
+                                      vals, vals2, nf, 0u, 63u, stream));
+  uint64_t* skeys = keys2;
+  uint32_t* svals = vals2;
 
-  BUILD_TRY(hipMemsetAsync(stats.p, 0, sizeof(uint32_t) * 4, stream));
-  DevBuf lbox, tbox, tcost, tcount, pos, offs, vals3, pleaf2;
+  BUILD_TRY(hipMemsetAsync(stats, 0, sizeof(uint32_t) * 4, stream));
   if (n >= 2) {
-    k_karras<<<blocks_for(ni), kBlock, 0, stream>>>(skeys, n, child.as<uint32_t>(), range.as<uint32_t>(),
-                                                    pint.as<int>(), pleaf.as<int>());
+    k_karras<<<blocks_for(ni), kBlock, 0, stream>>>(skeys, n, child, range,
+                                                    pint, pleaf);
     BUILD_TRY(hipGetLastError());
-    if (!(prm.flags & RMH_BVH_NO_REFINE) && n >= kTreeletLeaves) {
+    if (refine) {
       // SAH refinement of the radix tree, then depth-first leaf order so that every
       // subtree is again one range of the triangle array
-      BUILD_TRY(hipMalloc(&lbox.p, sizeof(float) * 6 * static_cast<size_t>(nf)));
-      BUILD_TRY(hipMalloc(&tbox.p, sizeof(float) * 6 * static_cast<size_t>(ni)));
-      BUILD_TRY(hipMalloc(&tcost.p, sizeof(float) * ni));
-      BUILD_TRY(hipMalloc(&tcount.p, sizeof(uint32_t) * ni));
-      BUILD_TRY(hipMalloc(&pos.p, sizeof(uint32_t) * nf));
-      BUILD_TRY(hipMalloc(&offs.p, sizeof(uint32_t) * ni));
-      BUILD_TRY(hipMalloc(&vals3.p, sizeof(uint32_t) * nf));
-      BUILD_TRY(hipMalloc(&pleaf2.p, sizeof(int) * nf));
       TreeArrays ta;
-      ta.child = child.as<uint32_t>();
-      ta.parent_int = pint.as<int>();
-      ta.parent_leaf = pleaf.as<int>();
-      ta.box = tbox.as<float>();
-      ta.cost = tcost.as<float>();
-      ta.count = tcount.as<uint32_t>();
-      ta.leaf_box = lbox.as<float>();
-      k_leaf_boxes<<<blocks_for(nf), kBlock, 0, stream>>>(nf, svals, flo.as<float4>(), fhi.as<float4>(), lbox.as<float>());
+      ta.child = child;
+      ta.parent_int = pint;
+      ta.parent_leaf = pleaf;
+      ta.box = tbox;
+      ta.cost = tcost;
+      ta.count = tcount;
+      ta.leaf_box = lbox;
+      k_leaf_boxes<<<blocks_for(nf), kBlock, 0, stream>>>(nf, svals, flo, fhi, lbox);
       BUILD_TRY(hipGetLastError());
-      BUILD_TRY(hipMemsetAsync(err.p, 0, sizeof(uint32_t), stream));
+      BUILD_TRY(hipMemsetAsync(err, 0, sizeof(uint32_t), stream));
       // triangle counts of the radix tree decide the first round's treelets; each round
       // leaves every count current for the next
-      k_range_counts<<<blocks_for(ni), kBlock, 0, stream>>>(ni, range.as<uint32_t>(), ta.count);
+      k_range_counts<<<blocks_for(ni), kBlock, 0, stream>>>(ni, range, ta.count);
       BUILD_TRY(hipGetLastError());
       for (int r = 0; r < kTreeletRounds; r++) {
         // the depths change with every round's restructuring
-        BUILD_TRY(make_levels(n, pint.as<int>(), ta.count, static_cast<uint32_t>(kTreeletLeaves), lb, err.as<uint32_t>(),
+        BUILD_TRY(make_levels(n, pint, ta.count, static_cast<uint32_t>(kTreeletLeaves), lb, err,
                               stream, levels));
         for (const LevelClass& c : levels) {
           if (c.treelet)
-            k_treelet_nodes<<<c.hi - c.lo, 64, 0, stream>>>(lb.order.as<uint32_t>(), c.lo, ta, prm.sah_cost_node,
+            k_treelet_nodes<<<c.hi - c.lo, 64, 0, stream>>>(lb.order, c.lo, ta, prm.sah_cost_node,
                                                             prm.sah_cost_tri);
           else
-            k_refresh_nodes<<<blocks_for(c.hi - c.lo), kBlock, 0, stream>>>(lb.order.as<uint32_t>(), c.lo, c.hi, ta,
+            k_refresh_nodes<<<blocks_for(c.hi - c.lo), kBlock, 0, stream>>>(lb.order, c.lo, c.hi, ta,
                                                                              prm.sah_cost_node, prm.sah_cost_tri);
           BUILD_TRY(hipGetLastError());
         }
       }
       {
-        DevBuf refs;
-        BUILD_TRY(hipMalloc(&refs.p, sizeof(uint32_t) * (2 * static_cast<size_t>(nf) - 1)));
-        BUILD_TRY(hipMemsetAsync(refs.p, 0, sizeof(uint32_t) * (2 * static_cast<size_t>(nf) - 1), stream));
-        k_check_tree<<<blocks_for(nf), kBlock, 0, stream>>>(n, ta, refs.as<uint32_t>(), err.as<uint32_t>());
+        BUILD_TRY(hipMemsetAsync(refs, 0, sizeof(uint32_t) * (2 * static_cast<size_t>(nf) - 1), stream));
+        k_check_tree<<<blocks_for(nf), kBlock, 0, stream>>>(n, ta, refs, err);
         BUILD_TRY(hipGetLastError());
-        k_check_refs<<<blocks_for(2 * static_cast<uint64_t>(nf)), kBlock, 0, stream>>>(n, refs.as<uint32_t>(),
-                                                                                       err.as<uint32_t>());
+        k_check_refs<<<blocks_for(2 * static_cast<uint64_t>(nf)), kBlock, 0, stream>>>(n, refs,
+                                                                                       err);
         BUILD_TRY(hipGetLastError());
         uint32_t terr = 0;
-        BUILD_TRY(hipMemcpyAsync(&terr, err.p, sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
+        BUILD_TRY(hipMemcpyAsync(&terr, err, sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
         BUILD_TRY(hipStreamSynchronize(stream));
         if (terr) { map_free(m); return fail(RMH_ERR_UNSUPPORTED, "rmh_map_build: BVH refinement produced an invalid tree"); }
       }
-      k_dfs_positions<<<blocks_for(nf), kBlock, 0, stream>>>(n, ta, pos.as<uint32_t>(), offs.as<uint32_t>());
+      k_dfs_positions<<<blocks_for(nf), kBlock, 0, stream>>>(n, ta, pos, offs);
       BUILD_TRY(hipGetLastError());
-      k_apply_order<<<blocks_for(nf), kBlock, 0, stream>>>(n, ta, pos.as<uint32_t>(), offs.as<uint32_t>(), svals,
-                                                           vals3.as<uint32_t>(), pleaf2.as<int>(), range.as<uint32_t>());
+      k_apply_order<<<blocks_for(nf), kBlock, 0, stream>>>(n, ta, pos, offs, svals,
+                                                           vals3, pleaf2, range);
       BUILD_TRY(hipGetLastError());
-      svals = vals3.as<uint32_t>();
-      std::swap(pleaf.p, pleaf2.p);
+      svals = vals3;
+      std::swap(pleaf, pleaf2);
     }
-    BUILD_TRY(make_levels(n, pint.as<int>(), nullptr, 0u, lb, err.as<uint32_t>(), stream, levels));
+    BUILD_TRY(make_levels(n, pint, nullptr, 0u, lb, err, stream, levels));
     for (const LevelClass& c : levels) {
       const uint32_t cnt = c.hi - c.lo;
-      k_bottom_up_level<<<blocks_for(cnt), kBlock, 0, stream>>>(lb.order.as<uint32_t>(), c.lo, c.hi, svals,
-                                                                flo.as<float4>(), fhi.as<float4>(), child.as<uint32_t>(),
-                                                                nlo.as<float4>(), nhi.as<float4>(), coll.as<uint8_t>(),
-                                                                subtree.as<uint32_t>(), prm.max_leaf_size,
+      k_bottom_up_level<<<blocks_for(cnt), kBlock, 0, stream>>>(lb.order, c.lo, c.hi, svals,
+                                                                flo, fhi, child,
+                                                                nlo, nhi, coll,
+                                                                subtree, prm.max_leaf_size,
                                                                 prm.sah_cost_node, prm.sah_cost_tri);
       BUILD_TRY(hipGetLastError());
     }
-    k_layout<<<std::min(blocks_for(ni), kWideBlocks), kBlock, 0, stream>>>(n, svals, flo.as<float4>(), fhi.as<float4>(), child.as<uint32_t>(),
-                                                    range.as<uint32_t>(), pint.as<int>(), nlo.as<float4>(),
-                                                    nhi.as<float4>(), coll.as<uint8_t>(), m->nodes, stats.as<uint32_t>(),
-                                                    m->reach);
+    k_layout<<<std::min(blocks_for(ni), kWideBlocks), kBlock, 0, stream>>>(n, svals, flo, fhi, child,
+                                                    range, pint, nlo,
+                                                    nhi, coll, slots, stats,
+                                                    reach);
     BUILD_TRY(hipGetLastError());
-    BUILD_TRY(hipMemcpyAsync(m->parent, pint.p, sizeof(int) * ni, hipMemcpyDeviceToDevice, stream));
   }
-  k_gather<<<blocks_for(nf), kBlock, 0, stream>>>(nf, svals, m->vertices, m->faces, moff.as<uint32_t>(), n_meshes,
+  k_gather<<<blocks_for(nf), kBlock, 0, stream>>>(nf, svals, m->vertices, m->faces, moff, n_meshes,
                                                   m->tris, m->normals);
   BUILD_TRY(hipGetLastError());
   BUILD_TRY(hipEventRecord(ev1, stream));
@@ -1367,10 +1416,10 @@ static int map_build(const float* vertices, uint32_t nv, const uint32_t* faces, 
   uint8_t root_collapsed = 0;
   float4 root_lo = make_float4(0, 0, 0, 0), root_hi = make_float4(0, 0, 0, 0);
   if (n >= 2) {
-    BUILD_TRY(hipMemcpy(hstats, stats.p, sizeof(hstats), hipMemcpyDeviceToHost));
-    BUILD_TRY(hipMemcpy(&root_collapsed, coll.p, 1, hipMemcpyDeviceToHost));
-    BUILD_TRY(hipMemcpy(&root_lo, nlo.p, sizeof(float4), hipMemcpyDeviceToHost));
-    BUILD_TRY(hipMemcpy(&root_hi, nhi.p, sizeof(float4), hipMemcpyDeviceToHost));
+    BUILD_TRY(hipMemcpy(hstats, stats, sizeof(hstats), hipMemcpyDeviceToHost));
+    BUILD_TRY(hipMemcpy(&root_collapsed, coll, 1, hipMemcpyDeviceToHost));
+    BUILD_TRY(hipMemcpy(&root_lo, nlo, sizeof(float4), hipMemcpyDeviceToHost));
+    BUILD_TRY(hipMemcpy(&root_hi, nhi, sizeof(float4), hipMemcpyDeviceToHost));
   }
   m->n_internal = ni;
   if (n == 1 || root_collapsed) {
@@ -1391,7 +1440,7 @@ static int map_build(const float* vertices, uint32_t nv, const uint32_t* faces, 
   }
   if (m->root == 0 && hstats[0] > 0) {
     BUILD_TRY(hipEventRecord(ev0, stream));
-    BUILD_TRY(preorder_nodes(m, ni, hstats[0], subtree.as<uint32_t>(), stream));
+    BUILD_TRY(preorder_nodes(m, ni, hstats[0], slots, pint, reach, subtree, rank, err, stream));
     BUILD_TRY(hipEventRecord(ev1, stream));
     BUILD_TRY(hipStreamSynchronize(stream));
     float order_ms = 0.0f;

@@ -40,8 +40,7 @@
 // costs a walk in an already coherent order more than it gains).  Each lane reads and writes
 // its own query's slots, so the results do not depend on the order.  Under stream capture,
 // or when the scratch cannot be had, the batch is walked in the caller's order.  The scratch
-// (17 B per query) comes from a pool of the library's own that keeps kPoolKeep bytes per
-// device between calls.
+// (17 B per query) comes from the library's pool (scratch_pool).
 #include "rmh_closest_bounds.hpp"
 #include "rmh_trace.hpp"
 
@@ -49,7 +48,6 @@
 
 #include <algorithm>
 #include <cfloat>
-#include <mutex>
 
 namespace {
 
@@ -323,32 +321,6 @@ __global__ __launch_bounds__(256) void k_order_spread(const rmh_vec3* q, const u
     const float v = part[threadIdx.x][0] + part[threadIdx.x][1] + part[threadIdx.x][2] + part[threadIdx.x][3];
     atomicAdd(&spread[threadIdx.x], v);
   }
-}
-
-// Stream-ordered pool of the sorting scratch, one per device, created at first use.  It keeps
-// up to kPoolKeep bytes after a synchronisation (the default pool would return them to the
-// driver, and map them again at the next call: 0.3 ms per call for 4M queries).
-constexpr uint64_t kPoolKeep = 256ull << 20;
-constexpr int kMaxPoolDevices = 64;
-
-hipMemPool_t scratch_pool(int device) {
-  static std::mutex mu;
-  static hipMemPool_t pools[kMaxPoolDevices] = {};
-  if (device < 0 || device >= kMaxPoolDevices) return nullptr;
-  std::lock_guard<std::mutex> lock(mu);
-  if (!pools[device]) {
-    hipMemPoolProps props = {};
-    props.allocType = hipMemAllocationTypePinned;
-    props.location.type = hipMemLocationTypeDevice;
-    props.location.id = device;
-    hipMemPool_t p = nullptr;
-    if (hipMemPoolCreate(&p, &props) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
-    uint64_t keep = kPoolKeep;
-    (void)hipMemPoolSetAttribute(p, hipMemPoolAttrReleaseThreshold, &keep);
-    (void)hipGetLastError();
-    pools[device] = p;
-  }
-  return pools[device];
 }
 
 // Morton order of the queries in `scratch` (stream-ordered; freed by the caller after the

@@ -12,6 +12,7 @@
 
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <new>
 #include <vector>
 
@@ -29,6 +30,29 @@ int fail(int code, const std::string& msg) {
 int hip_fail(hipError_t e, const char* what) {
   g_last_error = std::string("HIP error '") + hipGetErrorString(e) + "' in " + what;
   return RMH_ERR_HIP;
+}
+
+// With the default pool, whose memory is returned and mapped again around every
+// synchronisation, sorting 4M queries paid 0.3 ms more per call.
+hipMemPool_t scratch_pool(int device) {
+  constexpr int kMaxPoolDevices = 64;
+  static std::mutex mu;
+  static hipMemPool_t pools[kMaxPoolDevices] = {};
+  if (device < 0 || device >= kMaxPoolDevices) return nullptr;
+  std::lock_guard<std::mutex> lock(mu);
+  if (!pools[device]) {
+    hipMemPoolProps props = {};
+    props.allocType = hipMemAllocationTypePinned;
+    props.location.type = hipMemLocationTypeDevice;
+    props.location.id = device;
+    hipMemPool_t p = nullptr;
+    if (hipMemPoolCreate(&p, &props) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+    uint64_t keep = kPoolKeep;
+    (void)hipMemPoolSetAttribute(p, hipMemPoolAttrReleaseThreshold, &keep);
+    (void)hipGetLastError();
+    pools[device] = p;
+  }
+  return pools[device];
 }
 
 }  // namespace rmh
