@@ -203,7 +203,7 @@ def _events():
 
 def extra_batched(cpu_seconds: float, do_cpu: bool, tune: bool = True) -> dict:
     """Heterogeneous batch: 2,000 sensors (40 % VLP-16, 30 % pinhole 640x480, 30 % O1Dn with
-    1k-50k rays) on a 500k-triangle scene, hits + ranges, one persistent launch, tuned; the
+    1k-50k rays) on a 500k-triangle scene, hits + ranges, one launch, tuned; the
     split into two launches (image sensors, then ray lists) is timed beside it."""
     import torch
 
@@ -231,7 +231,7 @@ def extra_batched(cpu_seconds: float, do_cpu: bool, tune: bool = True) -> dict:
     batch.set_params(launches=1)
     batch.simulate()  # the parity check below reads the one-launch results
     layout = "4-wide" if tuned.get("wide") else "binary"
-    log(f"batched: {rays} rays, {ms:.2f} ms -> {rays / ms / 1e3:.1f} Mrays/s in one persistent launch "
+    log(f"batched: {rays} rays, {ms:.2f} ms -> {rays / ms / 1e3:.1f} Mrays/s in one launch "
         f"(two launches, images then ray lists: {split_ms:.2f} ms) (tuned {tuned['chunk_rays']}/"
         f"{tuned['waves_per_cu']}/{tuned['tile_rows']}, LDS stack {tuned['lds_stack']} {tuned['lds_stack_ms']}, "
         f"rays {'sorted' if tuned['rays_sorted'] else 'list order'} {tuned['ray_order_ms']}, {layout} nodes; "
@@ -257,9 +257,9 @@ def extra_batched(cpu_seconds: float, do_cpu: bool, tune: bool = True) -> dict:
     alg = 5 * rays + 12 * o1dn_rays + 32 * len(sensors)
     out = {"workload": f"{len(F)} tris (random boxes + icospheres, 200 m cube), {len(sensors)} sensors "
                        f"(800 VLP-16, 600 pinhole 640x480 fov 90, 600 O1Dn 1k-50k rays), hits+ranges",
-           "roofline": roofline("k_batch (one persistent launch, tuned)", alg, ms, BATCH_PROFILE,
+           "roofline": roofline("k_batch (one launch, tuned)", alg, ms, BATCH_PROFILE,
                                 "algorithmic bytes: hits + ranges (5 B/ray), O1Dn directions (12 B/ray), poses"),
-           "rays": rays, "launch": "one persistent launch", "batched_ms": round(ms, 3),
+           "rays": rays, "launch": "one launch", "batched_ms": round(ms, 3),
            "batched_mrays_s": round(rays / ms / 1e3, 1), "two_launches_ms": round(split_ms, 3),
            "per_sensor_launches_ms": round(plain_ms, 3), "per_sensor_mrays_s": round(rays / plain_ms / 1e3, 1),
            "tuned": {**{k: tuned[k] for k in ("chunk_rays", "waves_per_cu", "tile_rows", "lds_stack")},

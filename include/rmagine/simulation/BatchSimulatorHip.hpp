@@ -7,7 +7,7 @@
 // src/rmagine_core/include/rmagine/math/optimization.h:113-137).
 //
 //   BatchSimulatorHip  many simulators' sensor models, poses and result bundles, cast in one
-//                      persistent launch (rmh_batch_*); each bundle receives exactly what
+//                      launch (rmh_batch_*); each bundle receives exactly what
 //                      the simulator's own simulate() would write
 //   HipGraph           a recorded sequence of non-allocating librmh calls on one stream,
 //                      replayed with one call (rmh_graph_*)
@@ -26,8 +26,8 @@
 
 namespace rmagine {
 
-// rmh_batch_params; 0 keeps the current value (defaults: 256 rays per grab, 32 waves per
-// compute unit, 4 image rows per tile, 10 LDS stack rows, one persistent launch)
+// rmh_batch_params; 0 keeps the current value (defaults: 256 consecutive rays per XCD, 32
+// waves per compute unit, 4 image rows per tile, 10 LDS stack rows, one launch)
 struct BatchParamsHip {
   uint32_t chunk_rays = 0;
   uint32_t waves_per_cu = 0;

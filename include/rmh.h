@@ -279,8 +279,8 @@ int rmh_simulate_visit_stats(const rmh_map* map, const rmh_sensor* sensor, const
  * src/rmagine_optix/src/simulation/SphereSimulatorOptix.cpp:64-81; the closest piece is the
  * model union of src/rmagine_optix/include/rmagine/simulation/optix/sim_program_data.h:32-44).
  * A batch is a device table of sensors (any mix of models, poses and ray counts) cast in one
- * persistent launch (rmh_batch_params.launches = 2 splits it into image sensors, then O1Dn/OnDn
- * ray lists); every entry writes its own rmh_outputs exactly as rmh_simulate would. */
+ * launch (rmh_batch_params.launches = 2 splits it into image sensors, then O1Dn/OnDn ray
+ * lists); every entry writes its own rmh_outputs exactly as rmh_simulate would. */
 typedef struct {
   const rmh_sensor*    sensor;
   rmh_transform        Tsb;        /* sensor -> base (host value)               */
@@ -291,15 +291,17 @@ typedef struct {
 } rmh_batch_entry;
 
 typedef struct {
-  uint32_t chunk_rays;    /* rays per work grab, multiple of 64 (0 = keep / default 256)  */
-  uint32_t waves_per_cu;  /* persistent waves per compute unit (0 = keep / default 32)   */
+  uint32_t chunk_rays;    /* consecutive rays that go to one XCD, whose L2 serves them:
+                             multiple of 64 (0 = keep / default 256)                     */
+  uint32_t waves_per_cu;  /* most waves in flight per compute unit, of the 32 that fit
+                             (0 = keep / default 32; 1 counts as 2)                      */
   uint32_t tile_rows;     /* image rows per 64-ray tile of spherical/pinhole sensors:
                              1, 2, 4, 8, 16, 32 or 64, capped by the image height
                              (0 = keep / default 4)                                      */
   uint32_t lds_stack;     /* traversal stack entries per lane kept in LDS: 8, 10 or 16
                              (8 B each; 0 = keep / default 10); deeper entries go to
                              scratch                                                     */
-  uint32_t launches;      /* persistent launches per rmh_batch_simulate: 1 = every entry in
+  uint32_t launches;      /* launches per rmh_batch_simulate: 1 = every entry in
                              one launch (0 = keep / default), 2 = image sensors, then ray
                              lists, each kernel with its own walk                       */
 } rmh_batch_params;
@@ -313,9 +315,8 @@ int rmh_batch_create(const rmh_map* map, const rmh_batch_entry* entries, uint32_
 int rmh_batch_set_params(rmh_batch* batch, const rmh_batch_params* params);
 int rmh_batch_get_info(const rmh_batch* batch, uint64_t* total_rays, uint32_t* total_chunks,
                        rmh_batch_params* params);
-/* One counter-reset kernel + one persistent kernel on `stream` (per group when launches = 2,
- * in stream order); capturable into a graph.  Launches of one batch must not overlap (they
- * share its work counters). */
+/* One kernel on `stream` (one per group when launches = 2, in stream order); capturable into a
+ * graph.  Launches of one batch that overlap write the same outputs. */
 int rmh_batch_simulate(rmh_batch* batch, void* stream);
 int rmh_batch_destroy(rmh_batch* batch);
 

@@ -1,10 +1,10 @@
-"""Autotuner for the batched persistent launch (rmh_batch_*).
+"""Autotuner for the batched launch (rmh_batch_*).
 
-The persistent kernel has three launch parameters: rays handed out per work grab
-(`chunk_rays`, a multiple of 64), resident waves per compute unit (`waves_per_cu`, which
-sets the persistent grid) and the shape of the 64-ray tile a wave traces (`tile_rows` rows
+The batched kernel has three launch parameters: consecutive rays that go to one XCD
+(`chunk_rays`, a multiple of 64), waves in flight per compute unit (`waves_per_cu`, at most
+the 32 that fit) and the shape of the 64-ray tile a wave traces (`tile_rows` rows
 x 64/tile_rows columns of a spherical or pinhole image).  Small chunks balance uneven
-sensors better, large ones cost fewer atomics; more waves hide more latency until LDS and
+sensors better, large ones keep neighbouring rays in one L2; more waves hide more latency until LDS and
 registers run out; the tile shape decides how coherent a wave's rays are (on a spinning
 lidar wide tiles win because rays of one row end at similar ranges).  The tuner times
 every candidate on the caller's actual batch with HIP events and keeps the fastest:
@@ -12,7 +12,7 @@ first chunk x waves at the default tile, then the tile rows at the best pair, th
 depth of the traversal stack kept in LDS (`lds_stack`: 8, 10 or 16 rows of 8 B per ray; a
 shallower one leaves more LDS for resident waves, a deeper one spills less to private
 memory), then the ray order of the O1Dn/OnDn sensors (sorted by direction, or the list
-order the caller gave), then (when asked with launches=(1, 2)) one persistent launch for
+order the caller gave), then (when asked with launches=(1, 2)) one launch for
 every entry or two (image sensors, then ray lists, each kernel with its own walk), then
 (when asked with layouts=(False, True)) the BVH node layout of the batch's map: binary or
 4-wide with quantised boxes.  Stack depth, ray order, launch split and layout change speed,

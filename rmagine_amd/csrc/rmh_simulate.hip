@@ -22,12 +22,10 @@
 // Two launch forms:
 //   rmh_simulate        one sensor model, n poses, one workgroup per (pose, tile);
 //   rmh_batch_simulate  many sensors (any mix of models, poses and ray counts) in one
-//                       persistent launch (or, as a tuning choice, two: image sensors,
-//                       then ray lists, each with its own walk): waves grab chunks of tiles
-//                       of one sensor from an atomic counter until the work is exhausted.
-//                       All pointers and sizes live in a device table built once, so the
-//                       launch (counter reset kernel + persistent kernel) can be captured
-//                       into a graph.
+//                       launch (or, as a tuning choice, two: image sensors, then ray
+//                       lists, each with its own walk), one workgroup per tile of any
+//                       sensor.  All pointers and sizes live in a device table built once,
+//                       so the launch can be captured into a graph.
 // The reference has no batched form; its closest piece is the per-launch model union
 // (src/rmagine_optix/include/rmagine/simulation/optix/sim_program_data.h:32-44).
 #include "rmh_trace.hpp"
@@ -50,8 +48,7 @@ constexpr int kWave = 64;
 // through it after a traversal are scalar loads again (served by the scalar cache), where
 // the compiler would otherwise load the fields at the kernel's start and hold them in SGPRs
 // throughout: k_simulate's arguments outgrow the SGPRs, and the excess was spilled into VGPR
-// lanes, taking VGPRs from the traversal (terrain 8.80 -> 8.67 ms without them; the batched
-// kernel, whose entries live in device memory, measured slower with it and does not use it).
+// lanes, taking VGPRs from the traversal (terrain 8.80 -> 8.67 ms without them).
 // (The pointer is returned as a generic one; the cast from the constant address space stays
 // visible to the compiler, which reads through it with scalar loads.)
 template <class T>
@@ -212,16 +209,17 @@ struct BatchEntryDev {
   uint64_t n_slots;  // n_poses * tiles * 64 ray slots, enumerated tile by tile
 };
 
-// A persistent launch covers the entries [entry_lo, entry_hi), whose chunks are
-// [chunk_prefix[entry_lo], chunk_prefix[entry_hi]).
+// A launch covers the tiles [tile_lo, tile_lo + gridDim.x) of the entries [entry_lo, entry_hi);
+// entry i holds the tiles [tile_prefix[i], tile_prefix[i + 1]).
 struct BatchArgs {
   MapData map;
   const BatchEntryDev* entries;
-  const uint32_t* chunk_prefix;  // n_entries + 1
+  const uint64_t* tile_prefix;   // n_entries + 1
   uint32_t entry_lo, entry_hi;
-  uint32_t chunk_lo, chunk_hi;
-  uint32_t chunk_rays;           // multiple of 64
-  uint32_t* counter;
+  uint64_t tile_lo;
+  uint32_t run;                  // consecutive tiles one XCD receives
+  uint32_t dealt;                // tiles dealt in such runs: the launch's, rounded down to 8 runs
+  FastDiv div_run;
 };
 
 // Sensor-frame ray and map-frame ray of one slot of a batch entry.
@@ -250,84 +248,116 @@ __device__ __forceinline__ void with_kind(int kind, Fn&& fn) {
   fn(KindTag<RMH_MODEL_ONDN>{});
 }
 
-// One batch slot.  Ray generation and attribute writing depend on the sensor kind, the
+// One tile of a batch entry.  Ray generation and attribute writing depend on the sensor kind, the
 // traversal does not, so it is instantiated once per kernel (one copy of the
 // octant-specialised walks keeps the kernel inside the instruction cache).  As in
 // k_simulate, the ray set-up is recomputed for the writers rather than held (spilled)
-// through the traversal.
+// through the traversal: only the entry and tile indices are, and no register spills
+// (tile coordinates, the chunk loop's state and 64-bit bounds held as well: 9-17 SGPRs and
+// 7-15 VGPRs spilled, 30 mixed sensors x 16 poses 5.68 ms against 5.28).
 template <int STACK, int BLOCK, bool WIDE, int LDS, int SPEC>
-__device__ __forceinline__ void batch_ray(const BatchArgs& a, const BatchEntryDev* ep, int kind, uint32_t pose,
-                                          uint32_t tile, uint32_t vid, uint32_t hid, int2 (*stk)[BLOCK]) {
+__device__ __forceinline__ void batch_ray(const BatchArgs& a, uint32_t entry, uint32_t tg, int2 (*stk)[BLOCK]) {
   Hit h;
   {
-    const BatchEntryDev& e = *ep;
+    const BatchEntryDev& e = a.entries[entry];
+    const uint32_t pose = fast_div(tg, e.tl.div_tiles);
+    uint32_t vid, hid;
+    if (!tile_ray(e.tl, e.g.grid_w, e.g.grid_h, tg - pose * e.tl.tiles, threadIdx.x & 63u, vid, hid)) return;
+    const int kind = e.g.kind;
     const Tf Tsm = tmul(load_tf(e.Tbm[pose]), e.Tsb);
     uint32_t lid;
     V3 ds, os, dm, om;
     with_kind<SPEC>(kind, [&](auto k) { batch_gen<decltype(k)::value>(e, vid, hid, lid, Tsm, ds, os, dm, om); });
     trace<STACK, BLOCK, WIDE, SPEC, false, LDS>(a.map, om, dm, e.g.range_max, stk, h, speculative_walk(kind));
   }
-  // the entry's fields are read again after the traversal (the barrier hides that they are
-  // the same), and the ray's tile coordinates recomputed from the lane: holding either
-  // through the traversal spilled them to scratch once per tile
-  asm volatile("" : "+s"(ep));
+  // everything but the entry and tile indices is read again after the traversal (the
+  // barriers hide that it is the same)
   uint32_t lane = threadIdx.x & 63u;
   asm volatile("" : "+v"(lane));
-  const BatchEntryDev& e = *ep;
-  tile_ray(e.tl, e.g.grid_w, e.g.grid_h, tile, lane, vid, hid);
+  asm volatile("" : "+s"(entry), "+s"(tg));
+  const BatchArgs* ap = kernel_args<BatchArgs>();
+  const BatchEntryDev& e = ap->entries[entry];
+  const uint32_t pose = fast_div(tg, e.tl.div_tiles);
+  const int kind = e.g.kind;
+  uint32_t vid, hid;
+  tile_ray(e.tl, e.g.grid_w, e.g.grid_h, tg - pose * e.tl.tiles, lane, vid, hid);
   const Tf Tsm = tmul(load_tf(e.Tbm[pose]), e.Tsb);
   uint32_t lid;
   V3 ds, os;
   with_kind<SPEC>(kind, [&](auto k) { gen_ray<decltype(k)::value>(e.g, vid, hid, lid, ds, os); });
   const uint64_t r = static_cast<uint64_t>(pose) * e.g.ray_count + lid;
-  with_kind<SPEC>(kind, [&](auto k) { write_outputs<decltype(k)::value>(e.out, r, e.g, a.map, Tsm, ds, os, h); });
+  with_kind<SPEC>(kind, [&](auto k) { write_outputs<decltype(k)::value>(e.out, r, e.g, ap->map, Tsm, ds, os, h); });
 }
 
-__global__ void k_reset_counter(uint32_t* counter) {
-  if (threadIdx.x == 0) *counter = 0u;  // a kernel store (not a memset node) keeps graph replays correct
+// The entry that tile t belongs to: the last i in [lo, hi) with prefix[i] <= t.  64 bounds are
+// compared per step, one per lane (a binary search is a chain of log2(n) dependent loads at
+// the start of every workgroup).  Wave-uniform; every lane must be active.
+__device__ __forceinline__ uint32_t tile_entry(const uint64_t* prefix, uint32_t lo, uint32_t hi, uint64_t t) {
+  uint32_t n = hi - lo;  // prefix[lo] <= t < prefix[lo + n]
+  while (n > 1) {
+    const uint32_t step = (n + 63u) / 64u;
+    const uint32_t i = (threadIdx.x & 63u) * step;
+    const bool below = i < n && prefix[lo + i] <= t;
+    const uint32_t k = static_cast<uint32_t>(__popcll(__ballot(below))) - 1u;  // lane 0 is always below
+    n = __builtin_amdgcn_readfirstlane(n - k * step < step ? n - k * step : step);
+    lo = __builtin_amdgcn_readfirstlane(lo + k * step);
+  }
+  return lo;
 }
 
-// Persistent kernel over a range of entries.  SPEC = kSpecRuntime: every sensor kind in one
-// launch, ray lists walking speculatively and image sensors with the leaf holding switched
-// off; kSpecOff / kSpecOn: image sensors only (classic walk) / ray lists only, for a batch
-// cast as two launches.
+// The batched kernel over a range of entries, one workgroup per tile.  SPEC = kSpecRuntime:
+// every sensor kind in one launch, ray lists walking speculatively and image sensors with the
+// leaf holding switched off; kSpecOff / kSpecOn: image sensors only (classic walk) / ray lists
+// only.
+//
+// The hardware hands out the workgroups.  A persistent grid that took chunks of tiles from one
+// atomic counter was bound by that counter (11.7 ns per grab: 64-ray chunks of 49.9M rays 9.2
+// ms), so it took 256 rays at a time, which left the waves that met four scattered tiles in a
+// row running alone at the end; and its loop state, held through the traversal, spilled.  30
+// mixed sensors (40 % lidars, 30 % 640x480 cameras, 30 % ray lists) on 500k triangles: 16
+// poses (49.9M rays) 5.66 -> 5.28 ms, 2 poses 1.07 -> 0.77 ms.
 template <int STACK, int BLOCK, bool WIDE, int LDS, int SPEC>
 __global__ __launch_bounds__(BLOCK, 8) void k_batch(const BatchArgs a) {
   __shared__ int2 stk[LDS][BLOCK];
-  const int lane = threadIdx.x & 63;
-  for (;;) {
-    uint32_t c = 0;
-    if (lane == 0) c = atomicAdd(a.counter, 1u);
-    c = __shfl(c, 0, 64);
-    c = __builtin_amdgcn_readfirstlane(c) + a.chunk_lo;
-    if (c >= a.chunk_hi) break;  // every wave leaves once the counter passes the end
-    uint32_t lo = a.entry_lo, hi = a.entry_hi;
-    while (hi - lo > 1) {
-      const uint32_t mid = (lo + hi) >> 1;
-      if (a.chunk_prefix[mid] <= c) lo = mid; else hi = mid;
-    }
-    const BatchEntryDev& e = a.entries[lo];
-    const uint64_t tile0 = static_cast<uint64_t>(c - a.chunk_prefix[lo]) * (a.chunk_rays / 64);
-    const uint64_t n_tiles = static_cast<uint64_t>(e.n_poses) * e.tl.tiles;
-    const int kind = e.g.kind;
-    for (uint32_t k = 0; k < a.chunk_rays / 64; k++) {
-      if (tile0 + k >= n_tiles) break;
-      const uint32_t tg = static_cast<uint32_t>(tile0 + k);  // wave-uniform; n_tiles < 2^32
-      const uint32_t pose = fast_div(tg, e.tl.div_tiles);
-      const uint32_t tile = tg - pose * e.tl.tiles;
-      uint32_t vid, hid;
-      if (!tile_ray(e.tl, e.g.grid_w, e.g.grid_h, tile, lane, vid, hid)) continue;
-      batch_ray<STACK, BLOCK, WIDE, LDS, SPEC>(a, &e, kind, pose, tile, vid, hid, stk);
-    }
+  uint32_t b = blockIdx.x;
+  if (b < a.dealt) {  // workgroup b runs on XCD b % 8: runs of tiles dealt to the XCDs in turn
+    const uint32_t idx = b >> 3, round = fast_div(idx, a.div_run);
+    b = (round * 8u + (b & 7u)) * a.run + (idx - round * a.run);
   }
+  const uint64_t t = a.tile_lo + b;
+  // a captured launch replayed after the table was cut into other tiles may hold too many
+  if (t >= a.tile_prefix[a.entry_hi]) return;
+  const uint32_t entry = tile_entry(a.tile_prefix, a.entry_lo, a.entry_hi, t);
+  batch_ray<STACK, BLOCK, WIDE, LDS, SPEC>(a, entry, static_cast<uint32_t>(t - a.tile_prefix[entry]), stk);
 }
 
+// What one group of a batched launch casts: tiles [lo, hi) of the table, and how many waves may
+// share a compute unit.
+struct BatchSpan {
+  uint64_t lo, hi;
+  uint32_t waves_per_cu;
+};
+
+// Dynamic LDS that leaves `waves` one-wave workgroups of `used` bytes resident on a compute
+// unit (160 KB of LDS, handed out in steps of 1,280 bytes; a workgroup takes at most 64 KB,
+// so fewer than 2 cannot be asked for).
+uint32_t lds_padding(uint32_t waves, uint32_t used) {
+  const uint32_t share = std::min<uint32_t>(65536u, (160u * 1024u / waves) / 1280u * 1280u);
+  return share > used ? share - used : 0u;
+}
+
+// Tiles [lo, hi) of the table, in launches of at most kMaxTileBlocks.
 template <int STACK, bool WIDE, int LDS>
-hipError_t launch_batch(const BatchArgs& a, int spec, uint32_t blocks, hipStream_t stream) {
-  k_reset_counter<<<1, 64, 0, stream>>>(a.counter);
-  if (spec == kSpecRuntime) k_batch<STACK, kWave, WIDE, LDS, kSpecRuntime><<<blocks, kWave, 0, stream>>>(a);
-  else if (spec == kSpecOn) k_batch<STACK, kWave, WIDE, LDS, kSpecOn><<<blocks, kWave, 0, stream>>>(a);
-  else k_batch<STACK, kWave, WIDE, LDS, kSpecOff><<<blocks, kWave, 0, stream>>>(a);
+hipError_t launch_batch(BatchArgs a, int spec, const BatchSpan& span, hipStream_t stream) {
+  const uint32_t pad = lds_padding(span.waves_per_cu, sizeof(int2) * LDS * kWave);
+  for (uint64_t t = span.lo; t < span.hi; t += kMaxTileBlocks) {
+    const uint32_t blocks = static_cast<uint32_t>(std::min<uint64_t>(span.hi - t, kMaxTileBlocks));
+    a.tile_lo = t;
+    a.dealt = blocks / (8u * a.run) * (8u * a.run);
+    if (spec == kSpecRuntime) k_batch<STACK, kWave, WIDE, LDS, kSpecRuntime><<<blocks, kWave, pad, stream>>>(a);
+    else if (spec == kSpecOn) k_batch<STACK, kWave, WIDE, LDS, kSpecOn><<<blocks, kWave, pad, stream>>>(a);
+    else k_batch<STACK, kWave, WIDE, LDS, kSpecOff><<<blocks, kWave, pad, stream>>>(a);
+  }
   return hipGetLastError();
 }
 
@@ -335,22 +365,22 @@ hipError_t launch_batch(const BatchArgs& a, int spec, uint32_t blocks, hipStream
 // or 16 entries of 8 B per lane (4, 5 or 8 KiB per wave; 16 halves the resident waves);
 // deeper entries go to scratch.
 template <int STACK, bool WIDE>
-hipError_t launch_batch_lds(uint32_t lds, const BatchArgs& a, int spec, uint32_t blocks, hipStream_t stream) {
-  if (lds == 8) return launch_batch<STACK, WIDE, 8>(a, spec, blocks, stream);
-  if (lds == 16) return launch_batch<STACK, WIDE, 16>(a, spec, blocks, stream);
-  return launch_batch<STACK, WIDE, 10>(a, spec, blocks, stream);
+hipError_t launch_batch_lds(uint32_t lds, const BatchArgs& a, int spec, const BatchSpan& span, hipStream_t stream) {
+  if (lds == 8) return launch_batch<STACK, WIDE, 8>(a, spec, span, stream);
+  if (lds == 16) return launch_batch<STACK, WIDE, 16>(a, spec, span, stream);
+  return launch_batch<STACK, WIDE, 10>(a, spec, span, stream);
 }
 
-hipError_t launch_batch_sel(const TravSel& ts, uint32_t lds, const BatchArgs& a, int spec, uint32_t blocks,
-                            hipStream_t stream) {
+hipError_t launch_batch_sel(const TravSel& ts, uint32_t lds, const BatchArgs& a, int spec,
+                            const BatchSpan& span, hipStream_t stream) {
   if (ts.wide) {
-    if (ts.stack == 32) return launch_batch_lds<32, true>(lds, a, spec, blocks, stream);
-    if (ts.stack == 64) return launch_batch_lds<64, true>(lds, a, spec, blocks, stream);
-    return launch_batch_lds<128, true>(lds, a, spec, blocks, stream);
+    if (ts.stack == 32) return launch_batch_lds<32, true>(lds, a, spec, span, stream);
+    if (ts.stack == 64) return launch_batch_lds<64, true>(lds, a, spec, span, stream);
+    return launch_batch_lds<128, true>(lds, a, spec, span, stream);
   }
-  if (ts.stack == 32) return launch_batch_lds<32, false>(lds, a, spec, blocks, stream);
-  if (ts.stack == 64) return launch_batch_lds<64, false>(lds, a, spec, blocks, stream);
-  return launch_batch_lds<128, false>(lds, a, spec, blocks, stream);
+  if (ts.stack == 32) return launch_batch_lds<32, false>(lds, a, spec, span, stream);
+  if (ts.stack == 64) return launch_batch_lds<64, false>(lds, a, spec, span, stream);
+  return launch_batch_lds<128, false>(lds, a, spec, span, stream);
 }
 
 bool valid_lds_stack(uint32_t v) { return v == 8 || v == 10 || v == 16; }
@@ -360,15 +390,13 @@ bool valid_lds_stack(uint32_t v) { return v == 8 || v == 10 || v == 16; }
 struct rmh_batch {
   const rmh_map* map = nullptr;
   BatchEntryDev* entries = nullptr;
-  uint32_t* chunk_prefix = nullptr;
-  uint32_t* counter = nullptr;        // one work counter per launch group
+  uint64_t* tile_prefix = nullptr;
   uint32_t n_entries = 0;
   uint32_t n_image_entries = 0;       // the table holds the image entries first, then the ray lists
-  uint32_t image_chunks = 0;
-  uint32_t total_chunks = 0;
+  uint64_t image_tiles = 0, total_tiles = 0;
+  uint32_t total_chunks = 0;          // runs of chunk_rays rays, entry by entry
   uint64_t total_rays = 0;
   rmh_batch_params params{};
-  uint32_t n_cu = 256;
   std::vector<uint64_t> entry_rays;
   std::vector<BatchEntryDev> host;     // host copy of the table (re-tiled by set_params)
   std::vector<const rmh_sensor*> sensors;
@@ -379,8 +407,7 @@ namespace {
 void batch_free(rmh_batch* b) {
   if (!b) return;
   if (b->entries) (void)hipFree(b->entries);
-  if (b->chunk_prefix) (void)hipFree(b->chunk_prefix);
-  if (b->counter) (void)hipFree(b->counter);
+  if (b->tile_prefix) (void)hipFree(b->tile_prefix);
   delete b;
 }
 
@@ -398,20 +425,21 @@ void batch_tile(rmh_batch* b) {
   }
 }
 
+// Chunk count and tile prefix of the table, and the table itself unless `host` is empty.
 int batch_upload(rmh_batch* b, const std::vector<BatchEntryDev>& host) {
-  std::vector<uint32_t> prefix(b->n_entries + 1, 0);
+  std::vector<uint64_t> prefix(b->n_entries + 1, 0);
   uint64_t chunks = 0;
   for (uint32_t i = 0; i < b->n_entries; i++) {
     // the kernel enumerates an entry's tiles with 32-bit indices
     if (b->entry_rays[i] / 64u >= (1ull << 32)) return fail(RMH_ERR_UNSUPPORTED, "rmh_batch: an entry holds 2^32 or more ray tiles");
-    prefix[i] = static_cast<uint32_t>(chunks);
     chunks += (b->entry_rays[i] + b->params.chunk_rays - 1) / b->params.chunk_rays;
     if (chunks >= (1ull << 31)) return fail(RMH_ERR_UNSUPPORTED, "rmh_batch: too many ray chunks");
+    prefix[i + 1] = prefix[i] + b->entry_rays[i] / 64u;
   }
-  prefix[b->n_entries] = static_cast<uint32_t>(chunks);
   b->total_chunks = static_cast<uint32_t>(chunks);
-  b->image_chunks = prefix[b->n_image_entries];
-  RMH_HIP_TRY(hipMemcpy(b->chunk_prefix, prefix.data(), sizeof(uint32_t) * prefix.size(), hipMemcpyHostToDevice));
+  b->image_tiles = prefix[b->n_image_entries];
+  b->total_tiles = prefix[b->n_entries];
+  RMH_HIP_TRY(hipMemcpy(b->tile_prefix, prefix.data(), sizeof(uint64_t) * prefix.size(), hipMemcpyHostToDevice));
   if (!host.empty())
     RMH_HIP_TRY(hipMemcpy(b->entries, host.data(), sizeof(BatchEntryDev) * host.size(), hipMemcpyHostToDevice));
   return RMH_OK;
@@ -540,10 +568,6 @@ int rmh_batch_create(const rmh_map* map, const rmh_batch_entry* entries, uint32_
     batch_free(b);
     return fail(RMH_ERR_INVALID, "rmh_batch_create: launches must be 1 or 2");
   }
-  int dev = 0, ncu = 0;
-  (void)hipGetDevice(&dev);
-  if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && ncu > 0)
-    b->n_cu = static_cast<uint32_t>(ncu);
   b->host.resize(n_entries);
   b->sensors.resize(n_entries);
   b->entry_rays.resize(n_entries);
@@ -570,8 +594,7 @@ int rmh_batch_create(const rmh_map* map, const rmh_batch_entry* entries, uint32_
   }
   batch_tile(b);
   hipError_t err = hipMalloc(&b->entries, sizeof(BatchEntryDev) * std::max<uint32_t>(1, n_entries));
-  if (err == hipSuccess) err = hipMalloc(&b->chunk_prefix, sizeof(uint32_t) * (n_entries + 1));
-  if (err == hipSuccess) err = hipMalloc(&b->counter, 2 * sizeof(uint32_t));
+  if (err == hipSuccess) err = hipMalloc(&b->tile_prefix, sizeof(uint64_t) * (n_entries + 1));
   if (err != hipSuccess) { batch_free(b); return hip_fail(err, "rmh_batch_create"); }
   if (int rc = batch_upload(b, b->host)) { batch_free(b); return rc; }
   *out = b;
@@ -623,34 +646,28 @@ int rmh_batch_simulate(rmh_batch* b, void* stream_) {
   const TravSel ts = trav_select(b->map);
   if (ts.stack < 0) return fail(RMH_ERR_UNSUPPORTED, "rmh_batch_simulate: BVH deeper than 128 levels");
   hipStream_t stream = static_cast<hipStream_t>(stream_);
-  const uint32_t waves = b->n_cu * b->params.waves_per_cu;
   BatchArgs a;
   a.map = make_mapdata(b->map);
   a.entries = b->entries;
-  a.chunk_prefix = b->chunk_prefix;
-  a.chunk_rays = b->params.chunk_rays;
-  if (b->params.launches == 1) {
-    // one persistent launch over every entry (image entries first, then ray lists)
-    a.entry_lo = 0;
-    a.entry_hi = b->n_entries;
-    a.chunk_lo = 0;
-    a.chunk_hi = b->total_chunks;
-    a.counter = b->counter;
-    const uint32_t blocks = std::max<uint32_t>(1, std::min<uint32_t>(waves, b->total_chunks));
-    const hipError_t e = launch_batch_sel(ts, b->params.lds_stack, a, kSpecRuntime, blocks, stream);
-    if (e != hipSuccess) return hip_fail(e, "rmh_batch_simulate launch");
-    return RMH_OK;
-  }
-  // two persistent launches in stream order: the image entries, then the ray lists
-  for (int lists = 0; lists < 2; lists++) {
+  a.tile_prefix = b->tile_prefix;
+  a.tile_lo = 0;
+  a.dealt = 0;
+  a.run = b->params.chunk_rays / 64u;
+  a.div_run = make_fastdiv(a.run);
+  // one launch over every entry, or two in stream order: the image entries, then the ray lists.
+  // A batch of one kind takes the kernel of its kind in either case (9 cameras x 16 poses
+  // 4.26 -> 4.22 ms; the walk that serves both kinds keeps the speculative loop form).
+  const bool mixed = b->image_tiles > 0 && b->image_tiles < b->total_tiles;
+  const int groups = mixed && b->params.launches == 1 ? 1 : 2;
+  for (int k = 0; k < groups; k++) {
+    const bool lists = k == 1;
     a.entry_lo = lists ? b->n_image_entries : 0u;
-    a.entry_hi = lists ? b->n_entries : b->n_image_entries;
-    a.chunk_lo = lists ? b->image_chunks : 0u;
-    a.chunk_hi = lists ? b->total_chunks : b->image_chunks;
-    a.counter = b->counter + lists;
-    if (a.chunk_hi == a.chunk_lo) continue;
-    const uint32_t blocks = std::max<uint32_t>(1, std::min<uint32_t>(waves, a.chunk_hi - a.chunk_lo));
-    const hipError_t e = launch_batch_sel(ts, b->params.lds_stack, a, lists ? kSpecOn : kSpecOff, blocks, stream);
+    a.entry_hi = groups == 1 || lists ? b->n_entries : b->n_image_entries;
+    const BatchSpan span{lists ? b->image_tiles : 0u, groups == 1 || lists ? b->total_tiles : b->image_tiles,
+                         b->params.waves_per_cu};
+    if (span.lo == span.hi) continue;
+    const int spec = groups == 1 ? kSpecRuntime : (lists ? kSpecOn : kSpecOff);
+    const hipError_t e = launch_batch_sel(ts, b->params.lds_stack, a, spec, span, stream);
     if (e != hipSuccess) return hip_fail(e, "rmh_batch_simulate launch");
   }
   return RMH_OK;
