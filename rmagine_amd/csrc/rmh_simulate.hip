@@ -59,6 +59,17 @@ __device__ __forceinline__ const T* kernel_args() {
   return (const T*)p;
 }
 
+// Order of a plain cast over the XCDs.  Contiguous shares (each XCD its own poses) keep the
+// nodes around a pose in one L2, but an XCD whose poses are dear ends late: with few poses, or
+// where a pose's cost varies several times (a camera looks at much or at nothing), runs of 256
+// rays are dealt to the XCDs in turn instead.
+// Microseconds, contiguous / dealt: 60 and 200 cameras of 640x480 1,930 / 1,629 and 5,798 /
+// 5,246; 30 lidars of 128 x 1,024 on 2.1M triangles 693 / 586, 100 of them 1,140 / 1,133, 250
+// of them 2,234 / 2,273; 30 and 100 VLP-16 in a room 87 / 82 and 106.9 / 111.0.  Scattered
+// lists of which every XCD writes a part of each output line lose (256 lists of 32,768 rays
+// from one place, points, normals and hits: 2,530 / 2,690).
+constexpr uint32_t kWholePoses = 64, kDealRays = 256;
+
 struct SimArgs {
   MapData map;
   RayGen g;
@@ -66,9 +77,9 @@ struct SimArgs {
   const rmh_transform* Tbm;
   uint32_t pose_offset;              // first pose of this launch
   Tiling tl;
+  Deal deal;
   rmh_outputs out;
 };
-
 
 // Launch bounds ask for 8 waves per SIMD (64 VGPRs); with the writers' values recomputed or
 // re-read after the traversal, nothing spills (62-64 VGPRs, 62 SGPRs).
@@ -78,7 +89,7 @@ __global__ __launch_bounds__(kWave, 8) void k_simulate(const SimArgs a) {
   // block, pose and tile indices are wave-uniform: divided on the scalar unit, they stay in
   // SGPRs through the traversal instead of taking VGPRs (the scarce registers at 8 waves
   // per SIMD; `/` would run on the vector unit and leave its quotient there)
-  const uint32_t lb = xcd_contiguous(blockIdx.x, gridDim.x);
+  const uint32_t lb = xcd_deal(a.deal, blockIdx.x, gridDim.x);
   const uint32_t pl = fast_div(lb, a.tl.div_tiles);
   const uint32_t tile = lb - pl * a.tl.tiles;
   uint32_t vid, hid;
@@ -217,9 +228,7 @@ struct BatchArgs {
   const uint64_t* tile_prefix;   // n_entries + 1
   uint32_t entry_lo, entry_hi;
   uint64_t tile_lo;
-  uint32_t run;                  // consecutive tiles one XCD receives
-  uint32_t dealt;                // tiles dealt in such runs: the launch's, rounded down to 8 runs
-  FastDiv div_run;
+  Deal deal;                     // runs of chunk_rays rays, one XCD each
 };
 
 // Sensor-frame ray and map-frame ray of one slot of a batch entry.
@@ -319,23 +328,18 @@ __device__ __forceinline__ uint32_t tile_entry(const uint64_t* prefix, uint32_t 
 template <int STACK, int BLOCK, bool WIDE, int LDS, int SPEC>
 __global__ __launch_bounds__(BLOCK, 8) void k_batch(const BatchArgs a) {
   __shared__ int2 stk[LDS][BLOCK];
-  uint32_t b = blockIdx.x;
-  if (b < a.dealt) {  // workgroup b runs on XCD b % 8: runs of tiles dealt to the XCDs in turn
-    const uint32_t idx = b >> 3, round = fast_div(idx, a.div_run);
-    b = (round * 8u + (b & 7u)) * a.run + (idx - round * a.run);
-  }
-  const uint64_t t = a.tile_lo + b;
+  const uint64_t t = a.tile_lo + xcd_deal(a.deal, blockIdx.x, gridDim.x);
   // a captured launch replayed after the table was cut into other tiles may hold too many
   if (t >= a.tile_prefix[a.entry_hi]) return;
   const uint32_t entry = tile_entry(a.tile_prefix, a.entry_lo, a.entry_hi, t);
   batch_ray<STACK, BLOCK, WIDE, LDS, SPEC>(a, entry, static_cast<uint32_t>(t - a.tile_prefix[entry]), stk);
 }
 
-// What one group of a batched launch casts: tiles [lo, hi) of the table, and how many waves may
-// share a compute unit.
+// What one group of a batched launch casts: tiles [lo, hi) of the table in runs of `run` tiles
+// per XCD, and how many waves may share a compute unit.
 struct BatchSpan {
   uint64_t lo, hi;
-  uint32_t waves_per_cu;
+  uint32_t run, waves_per_cu;
 };
 
 // Dynamic LDS that leaves `waves` one-wave workgroups of `used` bytes resident on a compute
@@ -353,7 +357,7 @@ hipError_t launch_batch(BatchArgs a, int spec, const BatchSpan& span, hipStream_
   for (uint64_t t = span.lo; t < span.hi; t += kMaxTileBlocks) {
     const uint32_t blocks = static_cast<uint32_t>(std::min<uint64_t>(span.hi - t, kMaxTileBlocks));
     a.tile_lo = t;
-    a.dealt = blocks / (8u * a.run) * (8u * a.run);
+    a.deal = make_deal(blocks, span.run);
     if (spec == kSpecRuntime) k_batch<STACK, kWave, WIDE, LDS, kSpecRuntime><<<blocks, kWave, pad, stream>>>(a);
     else if (spec == kSpecOn) k_batch<STACK, kWave, WIDE, LDS, kSpecOn><<<blocks, kWave, pad, stream>>>(a);
     else k_batch<STACK, kWave, WIDE, LDS, kSpecOff><<<blocks, kWave, pad, stream>>>(a);
@@ -415,13 +419,17 @@ bool valid_tile_rows(uint32_t r) { return r >= 1 && r <= 64 && (r & (r - 1)) == 
 
 // Tiling, slot and ray counts of every entry for the batch's tile_rows.
 void batch_tile(rmh_batch* b) {
-  b->total_rays = 0;
+  uint64_t rays[2] = {0, 0};  // of the image entries, of the ray lists
+  for (uint32_t i = 0; i < b->n_entries; i++)
+    rays[i >= b->n_image_entries] += static_cast<uint64_t>(b->host[i].n_poses) * b->host[i].g.ray_count;
+  uint32_t lanes[2];
+  for (int k = 0; k < 2; k++) lanes[k] = rays_per_wave(rays[k], b->map->info.n_faces, k == 1);
+  b->total_rays = rays[0] + rays[1];
   for (uint32_t i = 0; i < b->n_entries; i++) {
     BatchEntryDev& h = b->host[i];
-    h.tl = sensor_tiling(b->sensors[i], b->params.tile_rows);
+    h.tl = sensor_tiling(b->sensors[i], b->params.tile_rows, lanes[i >= b->n_image_entries]);
     h.n_slots = static_cast<uint64_t>(h.n_poses) * h.tl.tiles * 64u;
     b->entry_rays[i] = h.n_slots;
-    b->total_rays += static_cast<uint64_t>(h.n_poses) * h.g.ray_count;
   }
 }
 
@@ -478,12 +486,16 @@ int rmh_simulate(const rmh_map* map, const rmh_sensor* sensor, const rmh_transfo
   a.out = *out;
   hipStream_t stream = static_cast<hipStream_t>(stream_);
 
-  a.tl = sensor_tiling(sensor);
+  const bool spec = sensor->speculative != 0;
+  const uint32_t lanes = rays_per_wave(ray_count * n_poses, map->info.n_faces, spec && speculative_walk(sensor->kind));
+  const bool dealt = n_poses < kWholePoses || sensor->kind == RMH_MODEL_PINHOLE;
+  a.tl = sensor_tiling(sensor, kDefaultTileRows, lanes);
   const uint32_t poses_per_launch = static_cast<uint32_t>(std::max<uint64_t>(1, kMaxTileBlocks / a.tl.tiles));
   for (uint32_t p0 = 0; p0 < n_poses; p0 += poses_per_launch) {
     const uint32_t np = std::min<uint32_t>(poses_per_launch, n_poses - p0);
     a.pose_offset = p0;
-    const hipError_t e = launch_sim(ts, sensor->kind, sensor->speculative != 0, a, np, stream);
+    a.deal = make_deal(np * a.tl.tiles, dealt ? kDealRays / lanes : 0u);
+    const hipError_t e = launch_sim(ts, sensor->kind, spec, a, np, stream);
     if (e != hipSuccess) return hip_fail(e, "rmh_simulate launch");
   }
   return RMH_OK;
@@ -651,9 +663,6 @@ int rmh_batch_simulate(rmh_batch* b, void* stream_) {
   a.entries = b->entries;
   a.tile_prefix = b->tile_prefix;
   a.tile_lo = 0;
-  a.dealt = 0;
-  a.run = b->params.chunk_rays / 64u;
-  a.div_run = make_fastdiv(a.run);
   // one launch over every entry, or two in stream order: the image entries, then the ray lists.
   // A batch of one kind takes the kernel of its kind in either case (9 cameras x 16 poses
   // 4.26 -> 4.22 ms; the walk that serves both kinds keeps the speculative loop form).
@@ -664,7 +673,7 @@ int rmh_batch_simulate(rmh_batch* b, void* stream_) {
     a.entry_lo = lists ? b->n_image_entries : 0u;
     a.entry_hi = groups == 1 || lists ? b->n_entries : b->n_image_entries;
     const BatchSpan span{lists ? b->image_tiles : 0u, groups == 1 || lists ? b->total_tiles : b->image_tiles,
-                         b->params.waves_per_cu};
+                         b->params.chunk_rays / 64u, b->params.waves_per_cu};
     if (span.lo == span.hi) continue;
     const int spec = groups == 1 ? kSpecRuntime : (lists ? kSpecOn : kSpecOff);
     const hipError_t e = launch_batch_sel(ts, b->params.lds_stack, a, spec, span, stream);

@@ -636,8 +636,8 @@ RMH_HD constexpr bool speculative_walk(int kind) { return kind == RMH_MODEL_O1DN
 template <int KIND>
 constexpr int spec_mode() { return speculative_walk(KIND) ? kSpecOn : kSpecOff; }
 
-// Ray tiles: each wave casts a th x tw block of one sensor image (th * tw = 64), which keeps
-// the 64 rays of a wave close in direction.  Tiles are 4 rows x 16 columns: rays of one
+// Ray tiles: each wave casts a th x tw block of one sensor image (th * tw = 64, or fewer: see
+// rays_per_wave), which keeps the rays of a wave close in direction.  Tiles are 4 rows x 16 columns: rays of one
 // row (same elevation for a spinning lidar) end at similar ranges, so wide tiles diverge
 // less than square ones (measured on the terrain: 4 x 16 is 7% faster than 8 x 8).
 // O1Dn/OnDn images of height 1 use 1 x 64.
@@ -649,12 +649,34 @@ struct Tiling {
 
 constexpr uint32_t kDefaultTileRows = 4;
 
-// rows: wanted tile height (a power of two <= 64), capped by the image height.
-inline Tiling make_tiling(uint32_t W, uint32_t H, uint32_t rows = kDefaultTileRows) {
+// Fewer rays per wave where 64 would leave the chip idle: a wave walks as long as the slowest
+// of its rays, and a launch of a few hundred waves ends with the slowest wave, while most of
+// the chip's 8,192 wave slots are empty.  Rays are split over more waves as long as half a
+// round of waves results; on a deep map (kDeepMap triangles or more: long walks, whose rays
+// differ most) two rounds, or for scattered lists (whose waves are long and uneven at any
+// size) 5/8 of one.  Measured, microseconds, 64 rays -> the rule's choice: 16 x 900 lidar in a
+// room (2,412 triangles) 1 pose 49 -> 36 (4 rays), 4 poses 54 -> 50 (16), 16 poses 63 (32 rays 62,
+// 16 rays 74; in a room of 25k triangles 48, 50 and 61); the lidar on 500k triangles 144 -> 65
+// (2); 128 x 1,024 lidar on 2.1M triangles 1 pose 222 -> 149 (8), 4 poses 358 -> 296 (32); 640 x 480
+// camera 206 -> 189 (16); 10,000 scattered rays 102 -> 67 (2), 16 lists 144 -> 140 (32; 16 rays
+// 156).
+constexpr uint32_t kDeepMap = 1u << 17;
+
+inline uint32_t rays_per_wave(uint64_t rays, uint32_t n_faces, bool scattered) {
+  const uint64_t most = n_faces < kDeepMap ? 4096u : (scattered ? 5120u : 16384u);
+  uint32_t lanes = 64;
+  while (lanes > 2 && rays / (lanes / 2) <= most) lanes /= 2;
+  return lanes;
+}
+
+// rows: wanted tile height (a power of two <= 64), capped by the image height; lanes: rays per
+// tile (a power of two).  Tiles of 2 and 4 rays have half as many rows.
+inline Tiling make_tiling(uint32_t W, uint32_t H, uint32_t rows = kDefaultTileRows, uint32_t lanes = 64u) {
   Tiling t;
   t.th = 1;
-  while (t.th * 2 <= rows && t.th * 2 <= H && t.th < 64) t.th *= 2;
-  t.tw = 64u / t.th;
+  const uint32_t most = lanes < 8u ? lanes / 2u : lanes;
+  while (t.th * 2 <= rows && t.th * 2 <= H && t.th < most) t.th *= 2;
+  t.tw = lanes / t.th;
   t.tiles_w = (W + t.tw - 1) / t.tw;
   t.tiles = t.tiles_w * ((H + t.th - 1) / t.th);
   t.tw_log2 = 0;
@@ -665,9 +687,9 @@ inline Tiling make_tiling(uint32_t W, uint32_t H, uint32_t rows = kDefaultTileRo
 }
 
 // Tiling of a sensor's image as the kernels cut it (ray lists: one row in traversal order).
-inline Tiling sensor_tiling(const rmh_sensor* s, uint32_t rows = kDefaultTileRows) {
+inline Tiling sensor_tiling(const rmh_sensor* s, uint32_t rows = kDefaultTileRows, uint32_t lanes = 64u) {
   const bool list = s->kind == RMH_MODEL_O1DN || s->kind == RMH_MODEL_ONDN;
-  return list ? make_tiling(s->width * s->height, 1u) : make_tiling(s->width, s->height, rows);
+  return list ? make_tiling(s->width * s->height, 1u, 1u, lanes) : make_tiling(s->width, s->height, rows, lanes);
 }
 
 // (row, column) of lane `lane` in tile `tile`; false for lanes outside the image.
@@ -691,6 +713,25 @@ __device__ __forceinline__ uint32_t xcd_dealt(uint32_t b, uint32_t n) {
   return (round * 8u + ((b + round) & 7u)) * S + (idx & (S - 1u));
 }
 
+// The same with the run length chosen at run time: 2^run_log2, for the first `dealt` indices.
+struct Deal {
+  uint32_t dealt, run_log2;
+};
+
+// run: indices per run, rounded down to a power of two; 0 = all contiguous
+inline Deal make_deal(uint32_t n, uint32_t run) {
+  Deal d{0u, 0u};
+  while ((2u << d.run_log2) <= run) d.run_log2++;
+  if (run) d.dealt = n >> (d.run_log2 + 3u) << (d.run_log2 + 3u);
+  return d;
+}
+
+__device__ __forceinline__ uint32_t xcd_deal(const Deal& d, uint32_t b, uint32_t n) {
+  if (b >= d.dealt) return d.dealt + xcd_contiguous(b - d.dealt, n - d.dealt);
+  const uint32_t idx = b >> 3, round = idx >> d.run_log2;
+  return (((round * 8u + ((b + round) & 7u)) - round) << d.run_log2) + idx;
+}
+
 // Most one-wave workgroups per launch of the (pose, tile) kernels: a dispatch holds the grid
 // size in work-items as a 32-bit count, so blocks x 64 stays below 2^31.
 constexpr uint64_t kMaxTileBlocks = 1ull << 25;
@@ -699,9 +740,10 @@ constexpr uint64_t kMaxTileBlocks = 1ull << 25;
 __device__ __forceinline__ bool tile_ray(const Tiling& t, uint32_t W, uint32_t H, uint32_t tile, uint32_t lane,
                                          uint32_t& vid, uint32_t& hid) {
   const uint32_t ty = fast_div(tile, t.div_tiles_w), tx = tile - ty * t.tiles_w;
-  vid = ty * t.th + (lane >> t.tw_log2);
+  const uint32_t row = lane >> t.tw_log2;
+  vid = ty * t.th + row;
   hid = tx * t.tw + (lane & (t.tw - 1u));
-  return vid < H && hid < W;
+  return row < t.th && vid < H && hid < W;
 }
 
 // Sensor-frame ray of tile coordinates (vid, hid) and its buffer index lid.  Spherical
