@@ -31,6 +31,7 @@
 // 131,072-point scan: 33 us of kernels with one butterfly per value, 64 blocks and one thread
 // per segment in the second pass, 10 us so; of one 16M-point cloud 540 and 170 us.
 #include "rmh_internal.hpp"
+#include "rmh_wave_sum.hpp"
 
 #include <cmath>
 #include <mutex>
@@ -166,61 +167,10 @@ __global__ void k_tf_pack_quat(const rmh_quat* q, const rmh_vec3* t, rmh_transfo
 
 // ---- reductions -------------------------------------------------------------------------
 
-template <int N>
-struct Acc {
-  double v[N];
-};
-
-// v and u of lanes 32 (or 16) apart, added crosswise: the lower of each pair gets the sum of
-// its own v and its partner's, the upper the sums of u (one swap instruction per word).
-__device__ __forceinline__ double swap_add32(double v, double u) {
-  const uint64_t a = __double_as_longlong(v), b = __double_as_longlong(u);
-  const auto lo = __builtin_amdgcn_permlane32_swap(static_cast<uint32_t>(a), static_cast<uint32_t>(b), false, false);
-  const auto hi = __builtin_amdgcn_permlane32_swap(static_cast<uint32_t>(a >> 32), static_cast<uint32_t>(b >> 32), false, false);
-  return __hiloint2double(static_cast<int>(hi[0]), static_cast<int>(lo[0])) +
-         __hiloint2double(static_cast<int>(hi[1]), static_cast<int>(lo[1]));
-}
-
-__device__ __forceinline__ double swap_add16(double v, double u) {
-  const uint64_t a = __double_as_longlong(v), b = __double_as_longlong(u);
-  const auto lo = __builtin_amdgcn_permlane16_swap(static_cast<uint32_t>(a), static_cast<uint32_t>(b), false, false);
-  const auto hi = __builtin_amdgcn_permlane16_swap(static_cast<uint32_t>(a >> 32), static_cast<uint32_t>(b >> 32), false, false);
-  return __hiloint2double(static_cast<int>(hi[0]), static_cast<int>(lo[0])) +
-         __hiloint2double(static_cast<int>(hi[1]), static_cast<int>(lo[1]));
-}
-
-// The same for any lane distance OFF, by one exchange of the half a lane does not keep.
-template <int OFF>
-__device__ __forceinline__ double cross_add(double v, double u) {
-  const bool up = (threadIdx.x & OFF) != 0;
-  return (up ? u : v) + __shfl_xor(up ? v : u, OFF, 64);
-}
-
-// Sums of N values over the wave, each left in the lanes of one group (value g in lanes
-// [g 64 / P, (g + 1) 64 / P), P the power of two from N): every step halves the values a lane
-// carries, so 16 values take 17 exchanges instead of the 96 of one butterfly per value.
-template <int N>
-__device__ __forceinline__ double wave_sum(const Acc<N>& a) {
-  constexpr int P = N <= 16 ? 16 : 32;
-  double v[P / 2];
-#pragma unroll
-  for (int k = 0; k < P / 2; k++) v[k] = swap_add32(k < N ? a.v[k] : 0.0, k + P / 2 < N ? a.v[k + P / 2] : 0.0);
-#pragma unroll
-  for (int k = 0; k < P / 4; k++) v[k] = swap_add16(v[k], v[k + P / 4]);
-#pragma unroll
-  for (int k = 0; k < P / 8; k++) v[k] = cross_add<8>(v[k], v[k + P / 8]);
-#pragma unroll
-  for (int k = 0; k < P / 16; k++) v[k] = cross_add<4>(v[k], v[k + P / 16]);
-  double x;
-  if constexpr (P == 32) x = cross_add<2>(v[0], v[1]);
-  else x = v[0] + __shfl_xor(v[0], 2, 64);
-  return x + __shfl_xor(x, 1, 64);
-}
-
 // Block-wide sums: left in lds[0] (every thread may read them on return).
 template <int N>
 __device__ __forceinline__ void block_sum(const Acc<N>& a, double (*lds)[N]) {
-  constexpr int G = N <= 16 ? 4 : 2;  // lanes per value
+  constexpr int G = N <= 8 ? 8 : (N <= 16 ? 4 : 2);  // lanes per value
   const double x = wave_sum(a);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   if (lane % G == 0 && lane / G < N) lds[w][lane / G] = x;

@@ -43,22 +43,6 @@ using namespace rmh;
 // occupancy follows the live waves instead of the slowest wave of a larger workgroup.
 constexpr int kWave = 64;
 
-// The launch arguments of a kernel whose only argument is a T, read through the kernarg
-// segment pointer (the argument starts the segment) hidden behind a barrier.  Reads made
-// through it after a traversal are scalar loads again (served by the scalar cache), where
-// the compiler would otherwise load the fields at the kernel's start and hold them in SGPRs
-// throughout: k_simulate's arguments outgrow the SGPRs, and the excess was spilled into VGPR
-// lanes, taking VGPRs from the traversal (terrain 8.80 -> 8.67 ms without them).
-// (The pointer is returned as a generic one; the cast from the constant address space stays
-// visible to the compiler, which reads through it with scalar loads.)
-template <class T>
-__device__ __forceinline__ const T* kernel_args() {
-  typedef const __attribute__((address_space(4))) T KArg;
-  KArg* p = (KArg*)__builtin_amdgcn_kernarg_segment_ptr();
-  asm volatile("" : "+s"(p));
-  return (const T*)p;
-}
-
 // Order of a plain cast over the XCDs.  Contiguous shares (each XCD its own poses) keep the
 // nodes around a pose in one L2, but an XCD whose poses are dear ends late: with few poses, or
 // where a pose's cost varies several times (a camera looks at much or at nothing), runs of 256
@@ -95,12 +79,12 @@ __global__ __launch_bounds__(kWave, 8) void k_simulate(const SimArgs a) {
   uint32_t vid, hid;
   if (!tile_ray(a.tl, a.g.grid_w, a.g.grid_h, tile, threadIdx.x, vid, hid)) return;
   const uint32_t pose = a.pose_offset + pl;
+  const Tf Tsm = uniform(tmul(load_tf(a.Tbm[pose]), a.Tsb));  // Tsm = Tbm * Tsb (SphereSimulatorEmbree.tcc:69-70)
   Hit h;
   {
     uint32_t lid;
     V3 ds, os;
     gen_ray<KIND>(a.g, vid, hid, lid, ds, os);
-    const Tf Tsm = tmul(load_tf(a.Tbm[pose]), a.Tsb);  // Tsm = Tbm * Tsb (SphereSimulatorEmbree.tcc:69-70)
     const V3 dm = qrot(Tsm.R, ds);
     const V3 om = map_origin<KIND>(Tsm, os);
     trace<STACK, kWave, WIDE, SPEC>(a.map, om, dm, a.g.range_max, stk, h);
@@ -113,7 +97,6 @@ __global__ __launch_bounds__(kWave, 8) void k_simulate(const SimArgs a) {
   uint32_t lid;
   V3 ds, os;
   gen_ray<KIND>(ap->g, vid, hid, lid, ds, os);
-  const Tf Tsm = tmul(load_tf(ap->Tbm[pose]), ap->Tsb);
   const uint64_t glob = static_cast<uint64_t>(pose) * ap->g.ray_count + lid;
   write_outputs<KIND>(ap->out, glob, ap->g, ap->map, Tsm, ds, os, h);
 }
@@ -267,13 +250,14 @@ __device__ __forceinline__ void with_kind(int kind, Fn&& fn) {
 template <int STACK, int BLOCK, bool WIDE, int LDS, int SPEC>
 __device__ __forceinline__ void batch_ray(const BatchArgs& a, uint32_t entry, uint32_t tg, int2 (*stk)[BLOCK]) {
   Hit h;
+  Tf Tsm;
   {
     const BatchEntryDev& e = a.entries[entry];
     const uint32_t pose = fast_div(tg, e.tl.div_tiles);
     uint32_t vid, hid;
     if (!tile_ray(e.tl, e.g.grid_w, e.g.grid_h, tg - pose * e.tl.tiles, threadIdx.x & 63u, vid, hid)) return;
     const int kind = e.g.kind;
-    const Tf Tsm = tmul(load_tf(e.Tbm[pose]), e.Tsb);
+    Tsm = uniform(tmul(load_tf(e.Tbm[pose]), e.Tsb));
     uint32_t lid;
     V3 ds, os, dm, om;
     with_kind<SPEC>(kind, [&](auto k) { batch_gen<decltype(k)::value>(e, vid, hid, lid, Tsm, ds, os, dm, om); });
@@ -290,7 +274,6 @@ __device__ __forceinline__ void batch_ray(const BatchArgs& a, uint32_t entry, ui
   const int kind = e.g.kind;
   uint32_t vid, hid;
   tile_ray(e.tl, e.g.grid_w, e.g.grid_h, tg - pose * e.tl.tiles, lane, vid, hid);
-  const Tf Tsm = tmul(load_tf(e.Tbm[pose]), e.Tsb);
   uint32_t lid;
   V3 ds, os;
   with_kind<SPEC>(kind, [&](auto k) { gen_ray<decltype(k)::value>(e.g, vid, hid, lid, ds, os); });

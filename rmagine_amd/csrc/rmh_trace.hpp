@@ -80,21 +80,39 @@ struct TriRay {
   int perm;  // 2 kz + swap (one register; the axes are derived at the leaves)
 };
 
+// x / z in FP64 for operands that are FP32 values, from y, an approximate 1 / z, with IEEE
+// rounding: with q = x y (1 + e1) and the exact residual x - z q, q + (x - z q) y misses x / z by
+// about e1 times the error of y, 2^-100 of it, before its one rounding.  A midpoint of two
+// doubles times z is not x (it has more bits than x), so the quotient lies at least 2^-78 of
+// itself away from every midpoint, and that rounding is the division's.  div_fixup gives
+// zeros, infinities and NaN their IEEE quotients.
+__device__ __forceinline__ double div_f32_f64(double x, double z, double y) {
+  const double q = x * y;
+  return __builtin_amdgcn_div_fixup(fma(fma(-z, q, x), y, q), z, x);
+}
+
+// One reciprocal serves the three quotients by the dominant component: 17 FP64 instructions
+// instead of 33, the same bits as three divisions.
 __device__ __forceinline__ TriRay make_tri_ray(const V3& o, const V3& d) {
   TriRay r;
   const float ax = fabsf(d.x), ay = fabsf(d.y), az = fabsf(d.z);
-  int kz = (ax > ay) ? (ax > az ? 0 : 2) : (ay > az ? 1 : 2);
-  int kx = kz == 2 ? 0 : kz + 1;
-  int ky = kx == 2 ? 0 : kx + 1;
-  const float dkz = kz == 0 ? d.x : (kz == 1 ? d.y : d.z);
-  if (dkz < 0.0f) { const int t = kx; kx = ky; ky = t; }
-  const double dd[3] = {(double)d.x, (double)d.y, (double)d.z};
-  const double oo[3] = {(double)o.x, (double)o.y, (double)o.z};
-  r.perm = 2 * kz + (dkz < 0.0f ? 1 : 0);
-  r.Sx = dd[kx] / dd[kz];
-  r.Sy = dd[ky] / dd[kz];
-  r.Sz = 1.0 / dd[kz];
-  r.okx = oo[kx]; r.oky = oo[ky]; r.okz = oo[kz];
+  // dominant axis z, else y, else x; the other two follow it cyclically
+  const bool kz0 = ax > ay && ax > az, kz1 = !(ax > ay) && ay > az;
+  const float dz = kz0 ? d.x : (kz1 ? d.y : d.z), oz = kz0 ? o.x : (kz1 ? o.y : o.z);
+  const float da = kz0 ? d.y : (kz1 ? d.z : d.x), oa = kz0 ? o.y : (kz1 ? o.z : o.x);
+  const float db = kz0 ? d.z : (kz1 ? d.x : d.y), ob = kz0 ? o.z : (kz1 ? o.x : o.y);
+  const bool swap = dz < 0.0f;
+  r.perm = (kz0 ? 0 : (kz1 ? 2 : 4)) + (swap ? 1 : 0);
+  const double z = dz;
+  double y = __builtin_amdgcn_rcp(z);
+  y = fma(fma(-z, y, 1.0), y, y);
+  y = fma(fma(-z, y, 1.0), y, y);
+  r.Sx = div_f32_f64(swap ? db : da, z, y);
+  r.Sy = div_f32_f64(swap ? da : db, z, y);
+  r.Sz = __builtin_amdgcn_div_fixup(fma(fma(-z, y, 1.0), y, y), z, 1.0);
+  r.okx = swap ? ob : oa;
+  r.oky = swap ? oa : ob;
+  r.okz = oz;
   return r;
 }
 
@@ -222,11 +240,12 @@ typedef __attribute__((address_space(1))) const int GInt;
 //   * P'' lies in [0.74 P, 1.26 P]: o +- P and its product with 1/d are rounded, at most
 //     2^-23 (|o| + P) <= P / 4 in position (the lo plane takes o + P, the hi plane o - P,
 //     so both planes move outward);
-//   * |r| <= 1.2e-7: the roundings of the reciprocal and of the fma.
+//   * |r| <= 1.8e-7: the error of the reciprocal instruction (1 ulp; the exactly rounded
+//     division takes ten instructions for the 0.5 ulp it saves) and the fma's rounding.
 // Replacing a direction component below 2^-64 by +-2^-64 moves the ray by at most
 // range_max 2^-64, far below P.  Let the exact ray meet the box at some t <= range_max in
 // [0, tbf] (tbf: an FP32 bound at least the closest hit found so far).  On each axis the near plane's exact crossing is <= t, so its moved
-// plane crosses at <= t - P''/|d| and the computed near value is <= t - P''/|d| + 1.2e-7 t
+// plane crosses at <= t - P''/|d| and the computed near value is <= t - P''/|d| + 1.8e-7 t
 // <= t, because P''/|d| >= 0.74 P >= 3.5e-7 range_max (|d| <= 1, t <= range_max); in the
 // same way every computed far value is >= t.  So tmin <= tmax holds as computed, with no
 // relative slack, and the box is never culled; boxes grow by about 2^-21 range_max
@@ -550,9 +569,9 @@ __device__ __forceinline__ void trace(const MapData& m, const V3& o, const V3& d
   if (m.n_faces == 0) return;
   constexpr float kMinDir = 0x1p-64f;
   SlabRay r;
-  r.idx = 1.0f / (fabsf(d.x) > kMinDir ? d.x : copysignf(kMinDir, d.x));
-  r.idy = 1.0f / (fabsf(d.y) > kMinDir ? d.y : copysignf(kMinDir, d.y));
-  r.idz = 1.0f / (fabsf(d.z) > kMinDir ? d.z : copysignf(kMinDir, d.z));
+  r.idx = __builtin_amdgcn_rcpf(fabsf(d.x) > kMinDir ? d.x : copysignf(kMinDir, d.x));
+  r.idy = __builtin_amdgcn_rcpf(fabsf(d.y) > kMinDir ? d.y : copysignf(kMinDir, d.y));
+  r.idz = __builtin_amdgcn_rcpf(fabsf(d.z) > kMinDir ? d.z : copysignf(kMinDir, d.z));
   const float omax = fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fabsf(o.z));
   const float P = (omax + range_max) * 0x1p-21f + 1e-30f;
   r.lx = -((o.x + P) * r.idx); r.hx = -((o.x - P) * r.idx);
@@ -735,6 +754,33 @@ __device__ __forceinline__ uint32_t xcd_deal(const Deal& d, uint32_t b, uint32_t
 // Most one-wave workgroups per launch of the (pose, tile) kernels: a dispatch holds the grid
 // size in work-items as a 32-bit count, so blocks x 64 stays below 2^31.
 constexpr uint64_t kMaxTileBlocks = 1ull << 25;
+
+// The launch arguments of a kernel whose only argument is a T, read through the kernarg
+// segment pointer (the argument starts the segment) hidden behind a barrier.  Reads made
+// through it after a traversal are scalar loads again (served by the scalar cache), where
+// the compiler would otherwise load the fields at the kernel's start and hold them in SGPRs
+// throughout: k_simulate's arguments outgrow the SGPRs, and the excess was spilled into VGPR
+// lanes, taking VGPRs from the traversal (terrain 8.80 -> 8.67 ms without them).
+// (The pointer is returned as a generic one; the cast from the constant address space stays
+// visible to the compiler, which reads through it with scalar loads.)
+template <class T>
+__device__ __forceinline__ const T* kernel_args() {
+  typedef const __attribute__((address_space(4))) T KArg;
+  KArg* p = (KArg*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return (const T*)p;
+}
+
+// A pose that is the same in all lanes, moved to scalar registers: 7 moves instead of the
+// pose product's ~60 vector instructions a second time for the attribute writers.
+__device__ __forceinline__ float uniform(float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); }
+
+__device__ __forceinline__ Tf uniform(const Tf& T) {
+  Tf r;
+  r.R.x = uniform(T.R.x); r.R.y = uniform(T.R.y); r.R.z = uniform(T.R.z); r.R.w = uniform(T.R.w);
+  r.t = v3(uniform(T.t.x), uniform(T.t.y), uniform(T.t.z));
+  return r;
+}
 
 // `tile` is wave-uniform in every caller, so its division stays on the scalar unit.
 __device__ __forceinline__ bool tile_ray(const Tiling& t, uint32_t W, uint32_t H, uint32_t tile, uint32_t lane,
