@@ -1033,7 +1033,8 @@ void map_free(rmh_map* m) {
   if (m->mesh_block) (void)hipFree(m->mesh_block);
   if (m->tree_block) (void)hipFree(m->tree_block);
   if (m->nodes4) (void)hipFree(m->nodes4);
-  if (m->refit_order) (void)hipFree(m->refit_order);
+  for (const RefitPass& r : m->refit_passes)
+    if (r.nodes) (void)hipFree(r.nodes);
   delete m;
 }
 
@@ -1534,87 +1535,198 @@ __device__ inline void set_child_box(Node2& nd, int c, float4 lo, float4 hi) {
   }
 }
 
-// Depth of every interior node of the final tree (0 at the root; unreachable slots get
-// UINT32_MAX).  The parent chain of a valid tree ends at the root.
-__global__ __launch_bounds__(kBlock) void k_node_depth(uint32_t ni, const uint8_t* __restrict__ reach,
-                                                       const int* __restrict__ parent, uint32_t* __restrict__ depth) {
-  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= ni) return;
-  if (!reach[i]) { depth[i] = 0xFFFFFFFFu; return; }
-  uint32_t d = 0;
-  for (int p = parent[i]; p >= 0; p = parent[p]) d++;
-  depth[i] = d;
-}
+// Box updates go bottom-up through the tree in a few passes.  Nodes lie in preorder, so of a
+// window of kWindow consecutive ones only the ancestors of the next window's first node have
+// anything below them outside the window: a chain of at most one node per level.  A pass gives
+// each window to one workgroup, which settles all its other nodes through the LDS; the
+// chains, a few per cent of the nodes and again a tree in preorder, are the next pass's
+// nodes.  1,048,576 vertices (one launch per level of the tree, 23 of them at 6.6 us, took
+// 150 us): see k_refit_window.
+constexpr uint32_t kWindow = 512;
 
-// One depth of the level-by-level refit: every node of the level boxes its two children,
-// leaf slots from their triangles, interior slots as the union of the child's own two
-// (already padded) boxes, refitted by the previous launch.  Each node is written by one
-// thread and read only by later launches, so no atomics or fences are needed (agent-scope
-// release and acquire write back and invalidate the L2 of an XCD on every such atomic,
-// which made the bottom-up pass with arrival counters 4 ms on the terrain).
-__global__ __launch_bounds__(kBlock) void k_refit_level(const uint32_t* __restrict__ order, uint32_t lo, uint32_t hi,
-                                                        const float4* __restrict__ tris, Node2* nodes) {
-  const uint32_t k = lo + blockIdx.x * kBlock + threadIdx.x;
-  if (k >= hi) return;
-  const uint32_t i = order[k];
-  Node2 nd = nodes[i];
-  for (int c = 0; c < 2; c++) {
-    const int ref = c ? nd.d.y : nd.d.x;
-    float4 blo, bhi;
-    if (ref < 0) {
-      const uint32_t e = ~static_cast<uint32_t>(ref);
-      const uint32_t first = e >> 3, cnt = (e & 7u) + 1u;
-      blo = make_float4(INFINITY, INFINITY, INFINITY, 0.0f);
-      bhi = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.0f);
-      for (uint32_t t = first; t < first + cnt; t++)
-        for (int v = 0; v < 3; v++) {
-          const float4 p = tris[3 * static_cast<size_t>(t) + v];
-          blo.x = fminf(blo.x, p.x); blo.y = fminf(blo.y, p.y); blo.z = fminf(blo.z, p.z);
-          bhi.x = fmaxf(bhi.x, p.x); bhi.y = fmaxf(bhi.y, p.y); bhi.z = fmaxf(bhi.z, p.z);
-        }
-    } else {
-      const Node2 ch = nodes[ref];
-      blo = make_float4(fminf(ch.a.x, ch.b.x), fminf(ch.a.z, ch.b.z), fminf(ch.c.x, ch.c.z), 0.0f);
-      bhi = make_float4(fmaxf(ch.a.y, ch.b.y), fmaxf(ch.a.w, ch.b.w), fmaxf(ch.c.y, ch.c.w), 0.0f);
-    }
-    set_child_box(nd, c, blo, bhi);
+// Lengths of the chains of a pass's windows, or (nodes given) the chains themselves, written at
+// the windows' offsets in preorder.  up[k]: position in the pass of node k's parent.
+__global__ __launch_bounds__(kBlock) void k_refit_chains(uint32_t n, const int* __restrict__ up, uint32_t* __restrict__ count,
+                                                         const uint32_t* __restrict__ offset,
+                                                         const uint32_t* __restrict__ from, uint32_t* __restrict__ nodes) {
+  const uint32_t w = blockIdx.x * kBlock + threadIdx.x;
+  if (static_cast<uint64_t>(w + 1) * kWindow >= n) return;  // nothing follows the last window
+  const int lo = static_cast<int>(w * kWindow);
+  uint32_t c = 0;
+  for (int p = up[lo + kWindow]; p >= lo; p = up[p]) {
+    if (nodes) nodes[offset[w + 1] - 1 - c] = from ? from[p] : static_cast<uint32_t>(p);
+    c++;
   }
-  nodes[i].a = nd.a;
-  nodes[i].b = nd.b;
-  nodes[i].c = nd.c;
+  if (count) count[w] = c;
 }
 
-// The refit schedule of a map (once: the tree's topology never changes after the build).
-hipError_t make_refit_schedule(rmh_map* m, hipStream_t stream) {
-  const uint32_t ni = m->n_internal;
-  uint32_t* depth = nullptr;
-  hipError_t e = hipMalloc(&depth, sizeof(uint32_t) * ni);
-  if (e != hipSuccess) return e;
-  k_node_depth<<<blocks_for(ni), kBlock, 0, stream>>>(ni, m->reach, m->parent, depth);
-  std::vector<uint32_t> hd(ni);
-  e = hipGetLastError();
-  if (e == hipSuccess) e = hipMemcpyAsync(hd.data(), depth, sizeof(uint32_t) * ni, hipMemcpyDeviceToHost, stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(stream);
-  (void)hipFree(depth);
-  if (e != hipSuccess) return e;
-  uint32_t max_d = 0, n = 0;
-  for (uint32_t d : hd)
-    if (d != 0xFFFFFFFFu) { max_d = std::max(max_d, d); n++; }
-  // counting sort, deepest level first
-  std::vector<uint32_t> start(max_d + 2, 0);
-  for (uint32_t d : hd)
-    if (d != 0xFFFFFFFFu) start[max_d - d + 1]++;
-  for (uint32_t l = 1; l < start.size(); l++) start[l] += start[l - 1];
-  std::vector<uint32_t> order(std::max<uint32_t>(1, n));
-  std::vector<uint32_t> fill(start.begin(), start.end() - 1);
-  for (uint32_t i = 0; i < ni; i++)
-    if (hd[i] != 0xFFFFFFFFu) order[fill[max_d - hd[i]]++] = i;
-  uint32_t* dev = nullptr;
-  e = hipMalloc(&dev, sizeof(uint32_t) * order.size());
-  if (e == hipSuccess) e = hipMemcpy(dev, order.data(), sizeof(uint32_t) * order.size(), hipMemcpyHostToDevice);
-  if (e != hipSuccess) { if (dev) (void)hipFree(dev); return e; }
-  m->refit_order = dev;
-  m->refit_levels = std::move(start);
+// Position of x in the ascending list, -1 if it is not there.
+__device__ __forceinline__ int list_position(const uint32_t* __restrict__ list, uint32_t n, uint32_t x) {
+  uint32_t lo = 0, hi = n;  // the first position whose value is >= x
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi) / 2;
+    if (list[mid] < x) lo = mid + 1; else hi = mid;
+  }
+  return lo < n && list[lo] == x ? static_cast<int>(lo) : -1;
+}
+
+// Children and parents of a pass's nodes as positions in the pass.
+__global__ __launch_bounds__(kBlock) void k_refit_links(uint32_t n, const uint32_t* __restrict__ list,
+                                                        const Node2* __restrict__ nodes, const int* __restrict__ parent,
+                                                        int* __restrict__ kids, int* __restrict__ up) {
+  const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+  if (k >= n) return;
+  const int4 d = nodes[list[k]].d;
+  kids[2 * k] = d.x < 0 ? -1 : list_position(list, n, static_cast<uint32_t>(d.x));
+  kids[2 * k + 1] = d.y < 0 ? -1 : list_position(list, n, static_cast<uint32_t>(d.y));
+  const int p = parent[list[k]];
+  up[k] = p < 0 ? -1 : list_position(list, n, static_cast<uint32_t>(p));
+}
+
+// Bounds of a leaf's triangles.
+__device__ __forceinline__ void leaf_box(const float4* __restrict__ tris, int ref, float4& lo, float4& hi) {
+  const uint32_t e = ~static_cast<uint32_t>(ref);
+  const uint32_t first = e >> 3, cnt = (e & 7u) + 1u;
+  lo = make_float4(INFINITY, INFINITY, INFINITY, 0.0f);
+  hi = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.0f);
+  for (uint32_t t = first; t < first + cnt; t++)
+    for (int v = 0; v < 3; v++) {
+      const float4 p = tris[3 * static_cast<size_t>(t) + v];
+      lo.x = fminf(lo.x, p.x); lo.y = fminf(lo.y, p.y); lo.z = fminf(lo.z, p.z);
+      hi.x = fmaxf(hi.x, p.x); hi.y = fmaxf(hi.y, p.y); hi.z = fmaxf(hi.z, p.z);
+    }
+}
+
+// Union of a node's two (already padded) boxes.
+__device__ __forceinline__ void union_box(const Node2& n, float4& lo, float4& hi) {
+  lo = make_float4(fminf(n.a.x, n.b.x), fminf(n.a.z, n.b.z), fminf(n.c.x, n.c.z), 0.0f);
+  hi = make_float4(fmaxf(n.a.y, n.b.y), fmaxf(n.a.w, n.b.w), fmaxf(n.c.y, n.c.w), 0.0f);
+}
+
+// One pass: a workgroup per window, a thread per node.  Leaf slots are boxed by the first pass
+// (FIRST) from their triangles; a child of an earlier pass is read from its node; the other
+// children are threads of the same workgroup, whose boxes go through the LDS round by round
+// until a round settles nothing.  Nodes left then have a child beyond the window: the next
+// pass holds exactly those.  The rounds cost barriers and LDS reads, not the memory latency
+// and launch that a level of the whole tree costs.
+template <bool FIRST>
+__global__ __launch_bounds__(kWindow) void k_refit_window(uint32_t n, const uint32_t* __restrict__ list,
+                                                          const int* __restrict__ kids, const float4* __restrict__ tris,
+                                                          Node2* nodes) {
+  __shared__ float box[6][kWindow];
+  __shared__ uint8_t ready[kWindow];
+  const uint32_t t = threadIdx.x, base = blockIdx.x * kWindow, k = base + t;
+  const uint32_t size = n - base < kWindow ? n - base : kWindow;
+  const bool mine = t < size;
+  ready[t] = 0;
+  Node2 nd;
+  uint32_t i = 0;
+  int wait[2] = {-1, -1};  // window positions of the children still to come
+  bool beyond = false;
+  if (mine) {
+    i = FIRST ? k : list[k];
+    nd = nodes[i];
+    for (int c = 0; c < 2; c++) {
+      const int ref = c ? nd.d.y : nd.d.x;
+      float4 lo, hi;
+      if (ref < 0) {
+        if constexpr (FIRST) {
+          leaf_box(tris, ref, lo, hi);
+          set_child_box(nd, c, lo, hi);
+        }
+        continue;
+      }
+      const int kid = FIRST ? ref : kids[2 * k + c];
+      if (kid < 0) {
+        union_box(nodes[ref], lo, hi);
+        set_child_box(nd, c, lo, hi);
+      } else if (static_cast<uint32_t>(kid) - base < size) {
+        wait[c] = kid - static_cast<int>(base);
+      } else {
+        beyond = true;
+      }
+    }
+  }
+  bool todo = mine && !beyond;
+  __syncthreads();
+  for (;;) {
+    if (todo) {
+      for (int c = 0; c < 2; c++)
+        if (wait[c] >= 0 && ready[wait[c]]) {
+          const int j = wait[c];
+          set_child_box(nd, c, make_float4(box[0][j], box[1][j], box[2][j], 0.0f),
+                        make_float4(box[3][j], box[4][j], box[5][j], 0.0f));
+          wait[c] = -1;
+        }
+    }
+    const bool settled = todo && wait[0] < 0 && wait[1] < 0;
+    if (!__syncthreads_or(settled)) break;  // also: every thread is done reading this round
+    if (settled) {
+      float4 lo, hi;
+      union_box(nd, lo, hi);
+      box[0][t] = lo.x; box[1][t] = lo.y; box[2][t] = lo.z;
+      box[3][t] = hi.x; box[4][t] = hi.y; box[5][t] = hi.z;
+      ready[t] = 1;
+      todo = false;
+    }
+    __syncthreads();
+  }
+  if (mine && (FIRST || (!todo && !beyond))) {
+    nodes[i].a = nd.a;
+    nodes[i].b = nd.b;
+    nodes[i].c = nd.c;
+  }
+}
+
+// The passes of a map (once: the tree's topology never changes after the build).
+hipError_t make_refit_passes(rmh_map* m, hipStream_t stream) {
+  std::vector<RefitPass> passes(1);
+  passes[0].n = m->n_internal;
+  int* up = nullptr;  // parent positions of the current pass; the first pass uses m->parent
+  uint32_t* lens = nullptr;
+  hipError_t e = hipMalloc(&lens, sizeof(uint32_t) * (2 * (m->n_internal / kWindow + 1) + 2));
+  while (e == hipSuccess && passes.back().n > kWindow) {
+    const RefitPass cur = passes.back();
+    const uint32_t nw = (cur.n + kWindow - 1) / kWindow;  // windows; the last has no chain
+    uint32_t* offs = lens + nw;
+    const int* cur_up = cur.nodes ? up : m->parent;
+    std::vector<uint32_t> h(nw), off(nw + 1, 0);
+    k_refit_chains<<<blocks_for(nw), kBlock, 0, stream>>>(cur.n, cur_up, lens, nullptr, cur.nodes, nullptr);
+    e = hipGetLastError();
+    if (e == hipSuccess) e = hipMemcpyAsync(h.data(), lens, sizeof(uint32_t) * (nw - 1), hipMemcpyDeviceToHost, stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(stream);
+    if (e != hipSuccess) break;
+    for (uint32_t w = 0; w + 1 < nw; w++) off[w + 1] = off[w] + h[w];
+    RefitPass next;
+    next.n = off[nw - 1];
+    if (next.n == 0 || next.n >= cur.n) { e = hipErrorInvalidValue; break; }  // a tree deeper than a window is wide
+    uint32_t* mem = nullptr;
+    int* next_up = nullptr;
+    e = hipMalloc(&mem, sizeof(uint32_t) * 3 * next.n);
+    if (e == hipSuccess) {
+      next.nodes = mem;
+      next.kids = reinterpret_cast<int*>(mem + next.n);
+      passes.push_back(next);
+      e = hipMalloc(&next_up, sizeof(int) * next.n);
+    }
+    if (e == hipSuccess) e = hipMemcpyAsync(offs, off.data(), sizeof(uint32_t) * nw, hipMemcpyHostToDevice, stream);
+    if (e == hipSuccess) {
+      k_refit_chains<<<blocks_for(nw), kBlock, 0, stream>>>(cur.n, cur_up, nullptr, offs, cur.nodes, next.nodes);
+      k_refit_links<<<blocks_for(next.n), kBlock, 0, stream>>>(next.n, next.nodes, m->nodes, m->parent, next.kids, next_up);
+      e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(stream);
+    if (up) (void)hipFree(up);
+    up = next_up;
+  }
+  if (up) (void)hipFree(up);
+  if (lens) (void)hipFree(lens);
+  if (e != hipSuccess) {
+    for (const RefitPass& r : passes)
+      if (r.nodes) (void)hipFree(r.nodes);
+    return e;
+  }
+  m->refit_passes = std::move(passes);
   return hipSuccess;
 }
 
@@ -1629,18 +1741,17 @@ extern "C" int rmh_map_refit(rmh_map* map, const float* vertices, void* stream_)
                                                                  map->normals);
   RMH_HIP_TRY(hipGetLastError());
   if (map->root >= 0 && map->n_internal > 0) {
-    if (!map->refit_order) {
-      const hipError_t e = make_refit_schedule(map, stream);
-      if (e != hipSuccess) return hip_fail(e, "rmh_map_refit: schedule");
+    if (map->refit_passes.empty()) {
+      const hipError_t e = make_refit_passes(map, stream);
+      if (e != hipSuccess) return hip_fail(e, "rmh_map_refit: passes");
     }
-    // one launch per depth, deepest first: a level reads only what earlier launches wrote
-    const std::vector<uint32_t>& lv = map->refit_levels;
+    // a pass reads only what earlier launches wrote, and its own window through the LDS
     hipError_t e = hipSuccess;
-    for (size_t l = 0; l + 1 < lv.size() && e == hipSuccess; l++) {
-      if (lv[l + 1] == lv[l]) continue;
-      k_refit_level<<<blocks_for(lv[l + 1] - lv[l]), kBlock, 0, stream>>>(map->refit_order, lv[l], lv[l + 1],
-                                                                           map->tris, map->nodes);
-      e = hipGetLastError();
+    for (const RefitPass& r : map->refit_passes) {
+      const uint32_t blocks = (r.n + kWindow - 1) / kWindow;
+      if (!r.nodes) k_refit_window<true><<<blocks, kWindow, 0, stream>>>(r.n, nullptr, nullptr, map->tris, map->nodes);
+      else k_refit_window<false><<<blocks, kWindow, 0, stream>>>(r.n, r.nodes, r.kids, map->tris, map->nodes);
+      if (e == hipSuccess) e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipStreamSynchronize(stream);
     if (e != hipSuccess) return hip_fail(e, "rmh_map_refit");

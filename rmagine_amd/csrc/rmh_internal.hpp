@@ -142,6 +142,15 @@ struct MapData {
   int root4;
 };
 
+// Nodes of one refit pass (see rmh_map_refit): n of them in preorder; `nodes` are their indices
+// and kids[2 k + c] the position in the pass of child c of its k-th node, -1 where that child
+// is a leaf or final already.  The first pass takes all nodes, and both are NULL.
+struct RefitPass {
+  uint32_t n = 0;
+  uint32_t* nodes = nullptr;
+  int* kids = nullptr;
+};
+
 }  // namespace rmh
 
 struct rmh_map {
@@ -168,11 +177,8 @@ struct rmh_map {
   rmh::Node4* nodes4 = nullptr;
   int root4 = 0;
   uint32_t wide_capacity = 0;          // allocated Node4 slots
-  // refit schedule, made at the first refit: the interior nodes of the final tree ordered by
-  // depth, deepest first, and where each depth starts (refit_levels[d] .. refit_levels[d+1]
-  // in reverse depth order)
-  uint32_t* refit_order = nullptr;
-  std::vector<uint32_t> refit_levels;
+  // refit passes, made at the first refit: the nodes that each pass leaves to the next
+  std::vector<rmh::RefitPass> refit_passes;
 };
 
 struct rmh_sensor {
