@@ -14,11 +14,13 @@
 //   uniform dust  d = min(r, max_range); with probability 1 - (1 - p_hit)^d a dust particle
 //                 at u * d is seen and returned with probability p_return^(u d): r = u d
 // n is a standard normal draw (Box-Muller, u1 in (0, 1], u2 in [0, 1)), u uniform; the
-// transcendental parts run in FP64 and round once to FP32.  cos(2 pi u2) comes from a
+// transcendental parts run in FP64 and round once to FP32.  sqrt(-2 log u1) is
+// normal_radius (rmh_noise_draw.hpp); cos(2 pi u2) comes from a
 // quadrant reduction in u2 (cos_2pi), r^1 is r, and the dust powers
 // of per-call bases are exp(y log base) with log base computed once on the host (pow's
 // x^0 = 1 kept): differences from pow far below the FP32 rounding of the result.
 #include "rmh_internal.hpp"
+#include "rmh_noise_draw.hpp"
 
 #include <cmath>
 
@@ -44,7 +46,6 @@ __device__ __forceinline__ U4 philox4x32_10(U4 c, uint32_t k0, uint32_t k1) {
   return c;
 }
 
-__device__ __forceinline__ double unit_open0(uint32_t x) { return (static_cast<double>(x >> 8) + 1.0) * 0x1p-24; }  // (0, 1]
 __device__ __forceinline__ double unit_open1(uint32_t x) { return static_cast<double>(x >> 8) * 0x1p-24; }          // [0, 1)
 
 struct NoiseArgs {
@@ -66,22 +67,22 @@ __device__ __forceinline__ double cos_2pi(double u) {
   const double x = (t - k) * 1.5707963267948966;
   const double x2 = x * x;
   double c = 1.0 / 20922789888000.0;          // 1/16!
-  c = fma(c, x2, -1.0 / 87178291200.0);       // 1/14!
-  c = fma(c, x2, 1.0 / 479001600.0);          // 1/12!
-  c = fma(c, x2, -1.0 / 3628800.0);           // 1/10!
-  c = fma(c, x2, 1.0 / 40320.0);              // 1/8!
-  c = fma(c, x2, -1.0 / 720.0);
-  c = fma(c, x2, 1.0 / 24.0);
+  c = fma_const(c, x2, -1.0 / 87178291200.0);       // 1/14!
+  c = fma_const(c, x2, 1.0 / 479001600.0);          // 1/12!
+  c = fma_const(c, x2, -1.0 / 3628800.0);           // 1/10!
+  c = fma_const(c, x2, 1.0 / 40320.0);              // 1/8!
+  c = fma_const(c, x2, -1.0 / 720.0);
+  c = fma_const(c, x2, 1.0 / 24.0);
   c = fma(c, x2, -0.5);
   c = fma(c, x2, 1.0);
   double sn = 1.0 / 355687428096000.0;        // 1/17!
-  sn = fma(sn, x2, -1.0 / 1307674368000.0);   // 1/15!
-  sn = fma(sn, x2, 1.0 / 6227020800.0);       // 1/13!
-  sn = fma(sn, x2, -1.0 / 39916800.0);        // 1/11!
-  sn = fma(sn, x2, 1.0 / 362880.0);           // 1/9!
-  sn = fma(sn, x2, -1.0 / 5040.0);
-  sn = fma(sn, x2, 1.0 / 120.0);
-  sn = fma(sn, x2, -1.0 / 6.0);
+  sn = fma_const(sn, x2, -1.0 / 1307674368000.0);   // 1/15!
+  sn = fma_const(sn, x2, 1.0 / 6227020800.0);       // 1/13!
+  sn = fma_const(sn, x2, -1.0 / 39916800.0);        // 1/11!
+  sn = fma_const(sn, x2, 1.0 / 362880.0);           // 1/9!
+  sn = fma_const(sn, x2, -1.0 / 5040.0);
+  sn = fma_const(sn, x2, 1.0 / 120.0);
+  sn = fma_const(sn, x2, -1.0 / 6.0);
   sn = fma(sn, x2, 1.0) * x;
   const int q = static_cast<int>(k) & 3;
   const double r = (q & 1) ? sn : c;
@@ -96,8 +97,14 @@ __device__ __forceinline__ double pow_from_log(double base, double log_base, dou
   return exp(y * log_base);
 }
 
-// One instantiation per model, so each carries only its own transcendentals (and registers).
-template <uint32_t KIND>
+// One instantiation per model, so each carries only its own transcendentals (and registers);
+// ANY_EXP: the relative model with an exponent other than 1, whose pow() takes 118 VGPRs and
+// with them half the resident waves.
+//
+// Bound by its instructions: 18 32-bit products of Philox and the FP64 parts (general log and
+// sqrt, constants through vector registers, pow() beside r^1 took 239 us for 32.8M relative
+// Gaussian ranges; 148 us now, of which moving the ranges takes 50 us).
+template <uint32_t KIND, bool ANY_EXP = false>
 __global__ __launch_bounds__(256) void k_noise(const NoiseArgs a) {
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
   for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < a.n; i += stride) {
@@ -113,10 +120,10 @@ __global__ __launch_bounds__(256) void k_noise(const NoiseArgs a) {
         if (unit_open1(w.z) < p_ret) a.r[i] = nr;
       }
     } else if (range <= a.max_range) {
-      const double n = sqrt(-2.0 * log(unit_open0(w.x))) * cos_2pi(unit_open1(w.y));
+      const double n = normal_radius((w.x >> 8) + 1u) * cos_2pi(unit_open1(w.y));
       double sd = static_cast<double>(a.b);
       if constexpr (KIND == RMH_NOISE_REL_GAUSSIAN)
-        sd *= a.c == 1.0f ? static_cast<double>(range) : pow(static_cast<double>(range), static_cast<double>(a.c));
+        sd *= ANY_EXP ? pow(static_cast<double>(range), static_cast<double>(a.c)) : static_cast<double>(range);
       a.r[i] = static_cast<float>(static_cast<double>(range) + n * sd + static_cast<double>(a.a));
     }
   }
@@ -148,7 +155,8 @@ extern "C" int rmh_noise_apply(const rmh_noise_params* params, float* ranges, ui
   const uint32_t blocks = static_cast<uint32_t>(want < 65536 ? want : 65536);
   const hipStream_t s = static_cast<hipStream_t>(stream);
   if (a.kind == RMH_NOISE_GAUSSIAN) k_noise<RMH_NOISE_GAUSSIAN><<<blocks, 256, 0, s>>>(a);
-  else if (a.kind == RMH_NOISE_REL_GAUSSIAN) k_noise<RMH_NOISE_REL_GAUSSIAN><<<blocks, 256, 0, s>>>(a);
+  else if (a.kind == RMH_NOISE_REL_GAUSSIAN && a.c == 1.0f) k_noise<RMH_NOISE_REL_GAUSSIAN><<<blocks, 256, 0, s>>>(a);
+  else if (a.kind == RMH_NOISE_REL_GAUSSIAN) k_noise<RMH_NOISE_REL_GAUSSIAN, true><<<blocks, 256, 0, s>>>(a);
   else k_noise<RMH_NOISE_UNIFORM_DUST><<<blocks, 256, 0, s>>>(a);
   RMH_HIP_TRY(hipGetLastError());
   return RMH_OK;
