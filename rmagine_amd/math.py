@@ -34,7 +34,7 @@ def _ptr(t) -> ctypes.c_void_p:
 def _check_dev(t, dtype, name, cols=None):
     if t is None:
         return
-    if not isinstance(t, torch.Tensor) or t.device.type != "cuda" or not t.is_contiguous() or t.dtype != dtype:
+    if not isinstance(t, torch.Tensor) or not t.is_cuda or not t.is_contiguous() or t.dtype != dtype:
         raise ValueError(f"{name} must be a contiguous {dtype} device tensor")
     if cols is not None and (t.dim() != 2 or t.shape[1] != cols):
         raise ValueError(f"{name} must have shape (N, {cols})")
@@ -55,8 +55,8 @@ class PointCloudView:
         _check_dev(self.mask, torch.uint8, "mask")
         _check_dev(self.ids, torch.int32, "ids")
         stride = segment_size if self.segment_stride is None else int(self.segment_stride)
-        return T.rmh_cloud(int(self.points.data_ptr()), _ptr(self.mask).value or 0, _ptr(self.normals).value or 0,
-                           _ptr(self.ids).value or 0, stride)
+        mask, normals, ids = (0 if t is None else t.data_ptr() for t in (self.mask, self.normals, self.ids))
+        return T.rmh_cloud(self.points.data_ptr(), mask, normals, ids, stride)
 
     def max_index(self, segment_size: int, n_segments: int) -> int:
         stride = segment_size if self.segment_stride is None else int(self.segment_stride)

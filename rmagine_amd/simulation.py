@@ -40,8 +40,11 @@ def _ptr(t) -> ctypes.c_void_p:
 
 
 def stream_handle(stream=None) -> ctypes.c_void_p:
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(int(s.cuda_stream))
+    # the current device's current stream without the Stream object that current_stream() makes
+    # (2.9 -> 0.4 us of every call; registering one scan makes two)
+    if stream is None:
+        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+    return ctypes.c_void_p(int(stream.cuda_stream))
 
 
 def _device_tensor(x, dtype, device) -> torch.Tensor:
