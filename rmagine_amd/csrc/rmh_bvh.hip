@@ -416,13 +416,14 @@ __global__ __launch_bounds__(kBlock) void k_leaf_boxes(uint32_t nf, const uint32
 }
 
 // One bottom-up treelet pass runs level by level over the current tree, deepest first
-// (make_levels): at each depth, k_refresh_nodes sets the box, count and cost of the nodes
-// with fewer than `gamma` triangles below from their children (thread per node), and
-// k_treelet_nodes does the same for the others and restructures each with one wave.  Children are final when their parent's level runs (earlier launches), a
-// treelet only involves nodes of its subtree, and the nodes of one depth have disjoint
-// subtrees, so no counters or fences are needed.  Which nodes get a treelet is known in
-// advance: a node's triangle count depends only on its leaf set, which restructuring below
-// it does not change.
+// (make_levels): at each depth, the box, count and cost of the nodes with fewer than `gamma`
+// triangles below are set from their children (thread per node), and those of the others
+// too, each of which one wave then restructures.  One launch does both (k_treelet_nodes);
+// k_refresh_nodes serves depths without treelets.  Children are final when their parent's
+// level runs (earlier launches), a treelet only involves nodes of its subtree, and the nodes
+// of one depth have disjoint subtrees, so no counters or fences are needed.  Which nodes get
+// a treelet is known in advance: a node's triangle count depends only on its leaf set, which
+// restructuring below it does not change.
 __global__ __launch_bounds__(kBlock) void k_refresh_nodes(const uint32_t* __restrict__ order, uint32_t lo, uint32_t hi,
                                                           TreeArrays t, float c_node, float c_tri) {
   const uint32_t k = lo + blockIdx.x * kBlock + threadIdx.x;
@@ -472,7 +473,7 @@ __device__ __forceinline__ float lane_f32(float v, uint32_t lane) {
   return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane));
 }
 
-// The seven-leaf treelet below every node of order[lo, lo + grid), one wave each: box, count
+// The seven-leaf treelet below every node of order[lo, mid), one wave each: box, count
 // and cost of the node from its children, then treelet_form, the dynamic program and
 // treelet_rebuild of rmh_treelet.hpp with the same choices and the same arithmetic (the trees
 // are those of the serial treelet_optimize()).  A node that gets a treelet has at least seven
@@ -487,12 +488,21 @@ __device__ __forceinline__ float lane_f32(float v, uint32_t lane) {
 // built in registers and its six nodes are written by six lanes.  With the treelet formed and
 // rebuilt by lane 0 through memory, and every subset's splits walked by one lane (126 steps
 // for the whole treelet), three rounds on the 2.1M-triangle terrain took 11.2 ms, 3.1 ms now.
-__global__ __launch_bounds__(64) void k_treelet_nodes(const uint32_t* __restrict__ order, uint32_t lo, TreeArrays t,
-                                                      float c_node, float c_tri) {
+//
+// The workgroups after those refresh the nodes order[mid, hi) of the same depth, 64 each: in a
+// launch of their own they took 8 us a depth and a gap (builds of 2.1M, 500k and 79k
+// triangles 5.64, 3.29 and 1.64 ms, now 5.43, 3.08 and 1.54).
+__global__ __launch_bounds__(64) void k_treelet_nodes(const uint32_t* __restrict__ order, uint32_t lo, uint32_t mid,
+                                                      uint32_t hi, TreeArrays t, float c_node, float c_tri) {
   static_assert(kTreeletLeaves == 7, "lanes are laid out for seven leaves");
   __shared__ float s_copt[128];
   __shared__ uint8_t s_part[128];
   const uint32_t lane = threadIdx.x;
+  if (blockIdx.x >= mid - lo) {
+    const uint32_t k = mid + (blockIdx.x - (mid - lo)) * 64u + lane;
+    if (k < hi) refresh_node(t, static_cast<int>(order[k]), c_node, c_tri);
+    return;
+  }
   const uint32_t root = __builtin_amdgcn_readfirstlane(order[lo + blockIdx.x]);
 
   // the treelet: lanes 0 and 1 start with the root's children; the interior leaf of largest
@@ -971,11 +981,10 @@ struct DevBuf {
 
 inline uint32_t blocks_for(uint64_t n) { return static_cast<uint32_t>((n + kBlock - 1) / kBlock); }
 
-// One launch range of the level-by-level passes: order[lo, hi) are nodes of one depth, with
-// or without a treelet.
+// One depth of the level-by-level passes: order[lo, mid) are its nodes with a treelet,
+// order[mid, hi) the others.
 struct LevelClass {
-  uint32_t lo, hi;
-  bool treelet;
+  uint32_t lo, mid, hi;
 };
 
 constexpr uint32_t kLevelKeys = 2u * (static_cast<uint32_t>(kMaxTreeWalk) + 1u);
@@ -1020,11 +1029,15 @@ hipError_t make_levels(int n, const int* parent_int, const uint32_t* count, uint
     return e;
   if ((e = hipStreamSynchronize(stream)) != hipSuccess) return e;
   classes.clear();
-  for (uint32_t k = 0; k < kLevelKeys; k++) {
-    if (st[k] == 0xFFFFFFFFu) continue;
-    if (!classes.empty()) classes.back().hi = st[k];
-    classes.push_back(LevelClass{st[k], ni, (k & 1u) == 0u});
+  uint32_t end = ni;
+  for (uint32_t d = kLevelKeys / 2u; d-- > 0;) {  // the keys are depth-major, so ranges end where the next begins
+    const uint32_t lo = st[2u * d], mid = st[2u * d + 1u];
+    if (lo == 0xFFFFFFFFu && mid == 0xFFFFFFFFu) continue;
+    const LevelClass c{lo != 0xFFFFFFFFu ? lo : mid, mid != 0xFFFFFFFFu ? mid : end, end};
+    classes.push_back(c);
+    end = c.lo;
   }
+  std::reverse(classes.begin(), classes.end());
   return hipSuccess;
 }
 
@@ -1360,9 +1373,9 @@ static int map_build(const float* vertices, uint32_t nv, const uint32_t* faces, 
         BUILD_TRY(make_levels(n, pint, ta.count, static_cast<uint32_t>(kTreeletLeaves), lb, err,
                               stream, levels));
         for (const LevelClass& c : levels) {
-          if (c.treelet)
-            k_treelet_nodes<<<c.hi - c.lo, 64, 0, stream>>>(lb.order, c.lo, ta, prm.sah_cost_node,
-                                                            prm.sah_cost_tri);
+          if (c.mid > c.lo)
+            k_treelet_nodes<<<c.mid - c.lo + (c.hi - c.mid + 63u) / 64u, 64, 0, stream>>>(
+                lb.order, c.lo, c.mid, c.hi, ta, prm.sah_cost_node, prm.sah_cost_tri);
           else
             k_refresh_nodes<<<blocks_for(c.hi - c.lo), kBlock, 0, stream>>>(lb.order, c.lo, c.hi, ta,
                                                                              prm.sah_cost_node, prm.sah_cost_tri);
