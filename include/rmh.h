@@ -180,7 +180,7 @@ int rmh_map_set_layout(rmh_map* map, int wide, void* stream);
  * positions and walked in that order when their order is spatially incoherent (random
  * points; not the rows of a scan); the results do not depend on the order.  The sort's
  * scratch (17 B per query) comes from a stream-ordered pool of the library that keeps up to
- * 256 MiB per device between calls; under stream capture the batch is walked as given. */
+ * 1 GiB per device between calls; under stream capture the batch is walked as given. */
 typedef struct {
   float* dist;
   rmh_vec3* points;
