@@ -44,14 +44,14 @@ using namespace rmh;
 constexpr int kWave = 64;
 
 // Order of a plain cast over the XCDs.  Contiguous shares (each XCD its own poses) keep the
-// nodes around a pose in one L2, but an XCD whose poses are dear ends late: with few poses, or
-// where a pose's cost varies several times (a camera over a deep map looks at much or at
+// nodes around a pose in one L2, but an XCD whose poses are dear ends late: over a deep map
+// with few poses, or where a pose's cost varies several times (a camera looks at much or at
 // nothing), runs of 256 rays are dealt to the XCDs in turn instead.
 // Microseconds, contiguous / dealt: 60 and 200 cameras of 640x480 1,930 / 1,629 and 5,798 /
 // 5,246; 30 lidars of 128 x 1,024 on 2.1M triangles 693 / 586, 100 of them 1,140 / 1,133, 250
-// of them 2,234 / 2,273; 30 and 100 VLP-16 in a room 87 / 82 and 106.9 / 111.0.  12 lidars of
-// 64 x 1,024 in a room 77.3 / 72.0.  Cameras in rooms are mixed (320 x 240, 8 poses 53.7 / 56.8 and
-// 46.0 / 47.5, 30 poses 111.2 / 102.5 and 99.5 / 100.4) and stay contiguous.  Scattered lists, of
+// of them 2,234 / 2,273.  Casts in rooms, whose map fits every L2, gain or lose: 12 lidars of
+// 64 x 1,024 77.3 / 72.0, 18 of 20 x 714 68.8 / 71.3, 100 VLP-16 106.9 / 111.0, 320 x 240 cameras, 8 poses
+// 53.7 / 56.8, 30 poses 111.2 / 102.5: they stay contiguous.  Scattered lists, of
 // which every XCD would write a part of each output line, lose (256 lists of 32,768 rays from
 // one place, points, normals and hits: 2,530 / 2,690; 30 lists of 20,000 in a room 90 / 100).
 constexpr uint32_t kWholePoses = 64, kDealRays = 256;
@@ -473,9 +473,9 @@ int rmh_simulate(const rmh_map* map, const rmh_sensor* sensor, const rmh_transfo
 
   const bool spec = sensor->speculative != 0;
   const bool scattered = spec && speculative_walk(sensor->kind);
-  const bool pinhole = sensor->kind == RMH_MODEL_PINHOLE, deep = map->info.n_faces >= kDeepMap;
   const uint32_t lanes = rays_per_wave(ray_count * n_poses, map->info.n_faces, scattered);
-  const bool dealt = !scattered && (pinhole ? deep : n_poses < kWholePoses);
+  const bool dealt = map->info.n_faces >= kDeepMap && !scattered &&
+                     (n_poses < kWholePoses || sensor->kind == RMH_MODEL_PINHOLE);
   a.tl = sensor_tiling(sensor, kDefaultTileRows, lanes);
   const uint32_t poses_per_launch = static_cast<uint32_t>(std::max<uint64_t>(1, kMaxTileBlocks / a.tl.tiles));
   for (uint32_t p0 = 0; p0 < n_poses; p0 += poses_per_launch) {
