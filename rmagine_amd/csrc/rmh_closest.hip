@@ -53,35 +53,6 @@ namespace {
 
 using namespace rmh;
 
-struct D3 { double x, y, z; };
-
-__device__ __forceinline__ D3 d3(double x, double y, double z) { D3 r; r.x = x; r.y = y; r.z = z; return r; }
-__device__ __forceinline__ D3 sub(const D3& a, const D3& b) { return d3(a.x - b.x, a.y - b.y, a.z - b.z); }
-__device__ __forceinline__ double ddot(const D3& a, const D3& b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
-__device__ __forceinline__ D3 madd(const D3& a, const D3& b, double s) { return d3(a.x + b.x * s, a.y + b.y * s, a.z + b.z * s); }
-
-// Closest point of triangle (a, b, c) to p.
-__device__ D3 closest_on_triangle(const D3& p, const D3& a, const D3& b, const D3& c) {
-  const D3 ab = sub(b, a), ac = sub(c, a), ap = sub(p, a);
-  const double d1 = ddot(ab, ap), d2 = ddot(ac, ap);
-  if (d1 <= 0.0 && d2 <= 0.0) return a;
-  const D3 bp = sub(p, b);
-  const double d3v = ddot(ab, bp), d4 = ddot(ac, bp);
-  if (d3v >= 0.0 && d4 <= d3v) return b;
-  const double vc = d1 * d4 - d3v * d2;
-  if (vc <= 0.0 && d1 >= 0.0 && d3v <= 0.0) return madd(a, ab, d1 / (d1 - d3v));
-  const D3 cp = sub(p, c);
-  const double d5 = ddot(ab, cp), d6 = ddot(ac, cp);
-  if (d6 >= 0.0 && d5 <= d6) return c;
-  const double vb = d5 * d2 - d1 * d6;
-  if (vb <= 0.0 && d2 >= 0.0 && d6 <= 0.0) return madd(a, ac, d2 / (d2 - d6));
-  const double va = d3v * d6 - d5 * d4;
-  if (va <= 0.0 && (d4 - d3v) >= 0.0 && (d5 - d6) >= 0.0)
-    return madd(b, sub(c, b), (d4 - d3v) / ((d4 - d3v) + (d5 - d6)));
-  const double den = 1.0 / (va + vb + vc);
-  return madd(madd(a, ab, vb * den), ac, vc * den);
-}
-
 struct CPArgs {
   MapData map;
   const rmh_vec3* q;
@@ -127,8 +98,9 @@ __global__ __launch_bounds__(64, 5) void k_closest(const CPArgs a) {
   // The walk runs on FP32 bounds: `upper` is at least the smallest squared distance met so
   // far (and at most about best0), and the triangles that may hold it are listed in LDS
   // (`cand`), to be evaluated in FP64 together at the end, or when the list is full.  A
-  // triangle is dropped only when its lower bound exceeds `upper`, so every triangle at the
-  // smallest FP64 distance is evaluated.
+  // triangle is dropped only when its lower bound exceeds `upper`, which only triangles shrink
+  // whose FP64 distance does not exceed it, so every triangle at the smallest FP64 distance is
+  // evaluated.
   double best = a.best0;
   uint32_t best_slot = 0xFFFFFFFFu, best_face = 0xFFFFFFFFu;
   float upper = upper_f32(best);

@@ -1,5 +1,6 @@
-// FP32 bounds of the closest-point walk (rmh_closest.hip), compiled for the device and, with
-// host stand-ins for the two approximate instructions, by tests/cpp/tri_bound_check.cpp.
+// Triangle distances of the closest-point walk (rmh_closest.hip): the FP64 evaluation and the
+// FP32 bounds, compiled for the device and, with host stand-ins for the two approximate
+// instructions, by tests/cpp/tri_bound_check.cpp and tests/cpp/closest_eval_check.cpp.
 #pragma once
 
 #include <cmath>
@@ -20,6 +21,35 @@
 #endif
 
 namespace rmh {
+
+struct D3 { double x, y, z; };
+
+RMH_CB_HD D3 d3(double x, double y, double z) { D3 r; r.x = x; r.y = y; r.z = z; return r; }
+RMH_CB_HD D3 sub(const D3& a, const D3& b) { return d3(a.x - b.x, a.y - b.y, a.z - b.z); }
+RMH_CB_HD double ddot(const D3& a, const D3& b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
+RMH_CB_HD D3 madd(const D3& a, const D3& b, double s) { return d3(a.x + b.x * s, a.y + b.y * s, a.z + b.z * s); }
+
+// Closest point of triangle (a, b, c) to p.
+RMH_CB_HD D3 closest_on_triangle(const D3& p, const D3& a, const D3& b, const D3& c) {
+  const D3 ab = sub(b, a), ac = sub(c, a), ap = sub(p, a);
+  const double d1 = ddot(ab, ap), d2 = ddot(ac, ap);
+  if (d1 <= 0.0 && d2 <= 0.0) return a;
+  const D3 bp = sub(p, b);
+  const double d3v = ddot(ab, bp), d4 = ddot(ac, bp);
+  if (d3v >= 0.0 && d4 <= d3v) return b;
+  const double vc = d1 * d4 - d3v * d2;
+  if (vc <= 0.0 && d1 >= 0.0 && d3v <= 0.0) return madd(a, ab, d1 / (d1 - d3v));
+  const D3 cp = sub(p, c);
+  const double d5 = ddot(ab, cp), d6 = ddot(ac, cp);
+  if (d6 >= 0.0 && d5 <= d6) return c;
+  const double vb = d5 * d2 - d1 * d6;
+  if (vb <= 0.0 && d2 >= 0.0 && d6 <= 0.0) return madd(a, ac, d2 / (d2 - d6));
+  const double va = d3v * d6 - d5 * d4;
+  if (va <= 0.0 && (d4 - d3v) >= 0.0 && (d5 - d6) >= 0.0)
+    return madd(b, sub(c, b), (d4 - d3v) / ((d4 - d3v) + (d5 - d6)));
+  const double den = 1.0 / (va + vb + vc);
+  return madd(madd(a, ab, vb * den), ac, vc * den);
+}
 
 struct F3 {
   float x, y, z;
@@ -55,9 +85,11 @@ RMH_CB_HD float walk_bound(float upper) { return fmaf(upper, 1.0f + 0x1p-19f, 1e
 //   products are off by three roundings each and by the vertices' rounding, together
 //   4.01 x 2^-24 |P|_1 M (|P|_1 the sum of P's components); 2^-21 of that is taken off.
 // Nothing is assumed of the choice of P: a poor one (overflow, NaN) only makes the lower bound
-// 0 and the upper one infinite or loose.  Slivers (sine of the angle at A below 0.003) and
-// values near the ends of the FP32 range get the lower bound 0, so that their FP64 evaluation
-// alone decides.
+// 0 and the upper one infinite or loose.  Degenerate triangles and slivers (sine of the angle at
+// A below 0.003) get the bounds 0 and infinity, so that their FP64 evaluation alone decides: it
+// has no result for equal A and B and queries on C's side (0 / 0), and in slivers its rounding
+// may exceed the margins, so an upper bound of theirs could drop the triangle that the
+// evaluation picks.  Values near the ends of the FP32 range get the lower bound 0.
 struct D2Bounds {
   float lo, hi;
 };
@@ -104,10 +136,11 @@ RMH_CB_HD D2Bounds triangle_bounds(const F3& A, const F3& B, const F3& C) {
   const float pp = fdot(P, P);
   const float m = fmaf(-lo_margin * (fabsf(P.x) + fabsf(P.y) + fabsf(P.z)), M, low), mm = m * m;
   const float u = fmaf(M, hi_margin, RMH_CB_SQRT(pp) * (1.0f + 0.5f * slack));
-  const bool plain = m > 0.0f && pp > 1e-30f && mm > 1e-30f && mm < 1e38f && fmaf(e, g, -(f * f)) > 1e-5f * (e * g);
+  const bool shaped = fmaf(e, g, -(f * f)) > 1e-5f * (e * g);
+  const bool plain = shaped && m > 0.0f && pp > 1e-30f && mm > 1e-30f && mm < 1e38f;
   D2Bounds r;
   r.lo = plain ? mm * RMH_CB_RCP(pp) * (1.0f - slack) : 0.0f;
-  r.hi = fmaf(u * u, 1.0f + slack, 1e-36f);
+  r.hi = shaped ? fmaf(u * u, 1.0f + slack, 1e-36f) : INFINITY;
   return r;
 }
 
