@@ -92,7 +92,8 @@ class BatchSimulatorHip {
     return rays;
   }
 
-  // asynchronous on the map's stream (or `stream`); launches of one batch must not overlap
+  // asynchronous on the map's stream (or `stream`); launches of one batch must not overlap, and
+  // graphs are captured again after a change of tile_rows
   void simulate() const { simulate(m_map->stream()); }
   void simulate(void* stream) const { RM_RMH_CHECK(rmh_batch_simulate(batch(), stream)); }
 

@@ -317,7 +317,10 @@ int rmh_batch_set_params(rmh_batch* batch, const rmh_batch_params* params);
 int rmh_batch_get_info(const rmh_batch* batch, uint64_t* total_rays, uint32_t* total_chunks,
                        rmh_batch_params* params);
 /* One kernel on `stream` (one per group when launches = 2, in stream order); capturable into a
- * graph.  Launches of one batch that overlap write the same outputs. */
+ * graph.  Launches of one batch that overlap write the same outputs.  A captured launch keeps the
+ * parameters and the number of tiles it was made with: after rmh_batch_set_params has changed
+ * tile_rows, capture again (a replay stays within the batch's poses and outputs, but leaves out
+ * the tiles beyond that number). */
 int rmh_batch_simulate(rmh_batch* batch, void* stream);
 int rmh_batch_destroy(rmh_batch* batch);
 

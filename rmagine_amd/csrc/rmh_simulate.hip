@@ -28,6 +28,7 @@
 //                       so the launch can be captured into a graph.
 // The reference has no batched form; its closest piece is the per-launch model union
 // (src/rmagine_optix/include/rmagine/simulation/optix/sim_program_data.h:32-44).
+#include "rmh_batch_tiles.hpp"
 #include "rmh_trace.hpp"
 
 #include <algorithm>
@@ -205,14 +206,14 @@ struct BatchEntryDev {
   uint64_t n_slots;  // n_poses * tiles * 64 ray slots, enumerated tile by tile
 };
 
-// A launch covers the tiles [tile_lo, tile_lo + gridDim.x) of the entries [entry_lo, entry_hi);
-// entry i holds the tiles [tile_prefix[i], tile_prefix[i + 1]).
+// A launch covers the tiles [tile_off, tile_off + gridDim.x) of the entries [entry_lo, entry_hi),
+// counted from their first; entry i holds the tiles [tile_prefix[i], tile_prefix[i + 1]).
 struct BatchArgs {
   MapData map;
   const BatchEntryDev* entries;
   const uint64_t* tile_prefix;   // n_entries + 1
   uint32_t entry_lo, entry_hi;
-  uint64_t tile_lo;
+  uint64_t tile_off;
   Deal deal;                     // runs of chunk_rays rays, one XCD each
 };
 
@@ -313,17 +314,17 @@ __device__ __forceinline__ uint32_t tile_entry(const uint64_t* prefix, uint32_t 
 template <int STACK, int BLOCK, bool WIDE, int LDS, int SPEC>
 __global__ __launch_bounds__(BLOCK, 8) void k_batch(const BatchArgs a) {
   __shared__ int2 stk[LDS][BLOCK];
-  const uint64_t t = a.tile_lo + xcd_deal(a.deal, blockIdx.x, gridDim.x);
-  // a captured launch replayed after the table was cut into other tiles may hold too many
-  if (t >= a.tile_prefix[a.entry_hi]) return;
+  // none for a recorded launch replayed after the table was cut into fewer tiles
+  uint64_t t;
+  if (!launch_tile(a.tile_prefix, a.entry_lo, a.entry_hi, a.tile_off + xcd_deal(a.deal, blockIdx.x, gridDim.x), t)) return;
   const uint32_t entry = tile_entry(a.tile_prefix, a.entry_lo, a.entry_hi, t);
   batch_ray<STACK, BLOCK, WIDE, LDS, SPEC>(a, entry, static_cast<uint32_t>(t - a.tile_prefix[entry]), stk);
 }
 
-// What one group of a batched launch casts: tiles [lo, hi) of the table in runs of `run` tiles
+// What one group of a batched launch casts: `tiles` tiles of its entries in runs of `run` tiles
 // per XCD, and how many waves may share a compute unit.
 struct BatchSpan {
-  uint64_t lo, hi;
+  uint64_t tiles;
   uint32_t run, waves_per_cu;
 };
 
@@ -335,13 +336,13 @@ uint32_t lds_padding(uint32_t waves, uint32_t used) {
   return share > used ? share - used : 0u;
 }
 
-// Tiles [lo, hi) of the table, in launches of at most kMaxTileBlocks.
+// The group's tiles, in launches of at most kMaxTileBlocks.
 template <int STACK, bool WIDE, int LDS>
 hipError_t launch_batch(BatchArgs a, int spec, const BatchSpan& span, hipStream_t stream) {
   const uint32_t pad = lds_padding(span.waves_per_cu, sizeof(int2) * LDS * kWave);
-  for (uint64_t t = span.lo; t < span.hi; t += kMaxTileBlocks) {
-    const uint32_t blocks = static_cast<uint32_t>(std::min<uint64_t>(span.hi - t, kMaxTileBlocks));
-    a.tile_lo = t;
+  for (uint64_t t = 0; t < span.tiles; t += kMaxTileBlocks) {
+    const uint32_t blocks = static_cast<uint32_t>(std::min<uint64_t>(span.tiles - t, kMaxTileBlocks));
+    a.tile_off = t;
     a.deal = make_deal(blocks, span.run);
     if (spec == kSpecRuntime) k_batch<STACK, kWave, WIDE, LDS, kSpecRuntime><<<blocks, kWave, pad, stream>>>(a);
     else if (spec == kSpecOn) k_batch<STACK, kWave, WIDE, LDS, kSpecOn><<<blocks, kWave, pad, stream>>>(a);
@@ -649,7 +650,6 @@ int rmh_batch_simulate(rmh_batch* b, void* stream_) {
   a.map = make_mapdata(b->map);
   a.entries = b->entries;
   a.tile_prefix = b->tile_prefix;
-  a.tile_lo = 0;
   // one launch over every entry, or two in stream order: the image entries, then the ray lists.
   // A batch of one kind takes the kernel of its kind in either case (9 cameras x 16 poses
   // 4.26 -> 4.22 ms; the walk that serves both kinds keeps the speculative loop form).
@@ -659,9 +659,9 @@ int rmh_batch_simulate(rmh_batch* b, void* stream_) {
     const bool lists = k == 1;
     a.entry_lo = lists ? b->n_image_entries : 0u;
     a.entry_hi = groups == 1 || lists ? b->n_entries : b->n_image_entries;
-    const BatchSpan span{lists ? b->image_tiles : 0u, groups == 1 || lists ? b->total_tiles : b->image_tiles,
-                         b->params.chunk_rays / 64u, b->params.waves_per_cu};
-    if (span.lo == span.hi) continue;
+    const uint64_t tiles = groups == 1 ? b->total_tiles : (lists ? b->total_tiles - b->image_tiles : b->image_tiles);
+    const BatchSpan span{tiles, b->params.chunk_rays / 64u, b->params.waves_per_cu};
+    if (span.tiles == 0) continue;
     const int spec = groups == 1 ? kSpecRuntime : (lists ? kSpecOn : kSpecOff);
     const hipError_t e = launch_batch_sel(ts, b->params.lds_stack, a, spec, span, stream);
     if (e != hipSuccess) return hip_fail(e, "rmh_batch_simulate launch");

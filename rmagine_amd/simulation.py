@@ -489,7 +489,8 @@ class BatchSimulatorHip:
         """Launch shape: consecutive rays per XCD, waves in flight per CU, image rows per 64-ray
         tile, traversal-stack entries held in LDS (8, 10 or 16; deeper entries spill to
         private memory), launches (1: every entry; 2: image sensors, then ray
-        lists) -- 0 keeps the current value."""
+        lists) -- 0 keeps the current value.  Capture graphs again after changing tile_rows: a
+        captured launch keeps the number of tiles it was made with."""
         prm = T.rmh_batch_params(chunk_rays, waves_per_cu, tile_rows, lds_stack, launches)
         _lib.call("rmh_batch_set_params", self._h, ctypes.byref(prm))
 
