@@ -6,6 +6,7 @@
 
 #include "rmh_fastdiv.hpp"
 #include "rmh_internal.hpp"
+#include "rmh_slab.hpp"
 
 namespace rmh {
 
@@ -233,28 +234,6 @@ typedef __attribute__((address_space(4))) const float CFloat;
 typedef __attribute__((address_space(1))) const char GChar;
 typedef __attribute__((address_space(1))) const float GFloat;
 typedef __attribute__((address_space(1))) const int GInt;
-
-// Slab test.  A slab value is fma(plane, 1/d, -(o +- P) / d) with a per-ray margin
-//   P = 2^-21 (max|o| + range_max) + 1e-30.
-// Written out, a computed value is t' = (plane - o -+ P'') / d * (1 + r), where
-//   * P'' lies in [0.74 P, 1.26 P]: o +- P and its product with 1/d are rounded, at most
-//     2^-23 (|o| + P) <= P / 4 in position (the lo plane takes o + P, the hi plane o - P,
-//     so both planes move outward);
-//   * |r| <= 1.8e-7: the error of the reciprocal instruction (1 ulp; the exactly rounded
-//     division takes ten instructions for the 0.5 ulp it saves) and the fma's rounding.
-// Replacing a direction component below 2^-64 by +-2^-64 moves the ray by at most
-// range_max 2^-64, far below P.  Let the exact ray meet the box at some t <= range_max in
-// [0, tbf] (tbf: an FP32 bound at least the closest hit found so far).  On each axis the near plane's exact crossing is <= t, so its moved
-// plane crosses at <= t - P''/|d| and the computed near value is <= t - P''/|d| + 1.8e-7 t
-// <= t, because P''/|d| >= 0.74 P >= 3.5e-7 range_max (|d| <= 1, t <= range_max); in the
-// same way every computed far value is >= t.  So tmin <= tmax holds as computed, with no
-// relative slack, and the box is never culled; boxes grow by about 2^-21 range_max
-// (0.05 mm at 100 m).  SlabRay holds the per-ray constants of that test.
-struct SlabRay {
-  float idx, idy, idz;   // reciprocal direction (components clamped away from zero)
-  float lx, ly, lz;      // -(o + P) / d: offsets of the lo planes
-  float hx, hy, hz;      // -(o - P) / d: offsets of the hi planes
-};
 
 // max(v, 0) and min(v, hi) of slab values as one v_med3_f32 each.  fminf/fmaxf would first
 // canonicalise an operand the compiler cannot prove canonical (tbf, which lives across the
@@ -567,16 +546,7 @@ __device__ __forceinline__ void trace(const MapData& m, const V3& o, const V3& d
   h.slot = 0xFFFFFFFFu;
   h.face = 0xFFFFFFFFu;
   if (m.n_faces == 0) return;
-  constexpr float kMinDir = 0x1p-64f;
-  SlabRay r;
-  r.idx = __builtin_amdgcn_rcpf(fabsf(d.x) > kMinDir ? d.x : copysignf(kMinDir, d.x));
-  r.idy = __builtin_amdgcn_rcpf(fabsf(d.y) > kMinDir ? d.y : copysignf(kMinDir, d.y));
-  r.idz = __builtin_amdgcn_rcpf(fabsf(d.z) > kMinDir ? d.z : copysignf(kMinDir, d.z));
-  const float omax = fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fabsf(o.z));
-  const float P = (omax + range_max) * 0x1p-21f + 1e-30f;
-  r.lx = -((o.x + P) * r.idx); r.hx = -((o.x - P) * r.idx);
-  r.ly = -((o.y + P) * r.idy); r.hy = -((o.y - P) * r.idy);
-  r.lz = -((o.z + P) * r.idz); r.hz = -((o.z - P) * r.idz);
+  const SlabRay r = make_slab_ray(o.x, o.y, o.z, d.x, d.y, d.z, range_max);
   // direction octant, specialised when the whole wave shares it (almost all tiles)
   const int oct = (r.idx < 0.0f ? 1 : 0) | (r.idy < 0.0f ? 2 : 0) | (r.idz < 0.0f ? 4 : 0);
   const int oct0 = __builtin_amdgcn_readfirstlane(oct);
