@@ -292,8 +292,9 @@ typedef struct {
 
 typedef struct {
   uint32_t chunk_rays;    /* consecutive rays that go to one XCD, whose L2 serves them:
-                             multiple of 64, cast in runs of the next lower power of
-                             two (0 = keep / default 256)                                */
+                             multiple of 64, cast in runs of chunk_rays / 64 tiles,
+                             rounded down to a power of two (a tile holds 64 rays,
+                             fewer in batches of few rays; 0 = keep / default 256)       */
   uint32_t waves_per_cu;  /* most waves in flight per compute unit, of the 32 that fit
                              (0 = keep / default 32; 1 counts as 2)                      */
   uint32_t tile_rows;     /* image rows per 64-ray tile of spherical/pinhole sensors:
