@@ -98,12 +98,12 @@ __device__ __forceinline__ double pow_from_log(double base, double log_base, dou
 }
 
 // One instantiation per model, so each carries only its own transcendentals (and registers);
-// ANY_EXP: the relative model with an exponent other than 1, whose pow() takes 118 VGPRs and
-// with them half the resident waves.
+// ANY_EXP: the relative model with an exponent other than 1, whose pow() takes 83 VGPRs (34
+// without it), which leaves five waves per SIMD.
 //
 // Bound by its instructions: 18 32-bit products of Philox and the FP64 parts (general log and
 // sqrt, constants through vector registers, pow() beside r^1 took 239 us for 32.8M relative
-// Gaussian ranges; 148 us now, of which moving the ranges takes 50 us).
+// Gaussian ranges; 155 us now, of which moving the ranges takes 50 us).
 template <uint32_t KIND, bool ANY_EXP = false>
 __global__ __launch_bounds__(256) void k_noise(const NoiseArgs a) {
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
