@@ -1764,7 +1764,7 @@ extern "C" int rmh_map_refit(rmh_map* map, const float* vertices, void* stream_)
       const uint32_t blocks = (r.n + kWindow - 1) / kWindow;
       if (!r.nodes) k_refit_window<true><<<blocks, kWindow, 0, stream>>>(r.n, nullptr, nullptr, map->tris, map->nodes);
       else k_refit_window<false><<<blocks, kWindow, 0, stream>>>(r.n, r.nodes, r.kids, map->tris, map->nodes);
-      if (e == hipSuccess) e = hipGetLastError();
+      if ((e = hipGetLastError()) != hipSuccess) break;
     }
     if (e == hipSuccess) e = hipStreamSynchronize(stream);
     if (e != hipSuccess) return hip_fail(e, "rmh_map_refit");
