@@ -334,13 +334,12 @@ __global__ __launch_bounds__(kBlock) void k_preorder_rank(uint32_t ni, const uin
   rank[i] = r;
 }
 
-// 8b: move every reachable node to its preorder slot, with its child references, parent
-// link and reach flag renumbered.
+// 8b: move every reachable node to its preorder slot, with its child references and parent link
+// renumbered.
 __global__ __launch_bounds__(kBlock) void k_preorder_scatter(uint32_t ni, uint32_t n_out, const uint8_t* __restrict__ reach,
                                                              const int* __restrict__ parent, const Node2* __restrict__ nodes,
                                                              const uint32_t* __restrict__ rank, Node2* __restrict__ out,
-                                                             int* __restrict__ out_parent, uint8_t* __restrict__ out_reach,
-                                                             uint32_t* err) {
+                                                             int* __restrict__ out_parent, uint32_t* err) {
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= ni || !reach[i]) return;
   const uint32_t s = rank[i];
@@ -350,7 +349,6 @@ __global__ __launch_bounds__(kBlock) void k_preorder_scatter(uint32_t ni, uint32
   if (nd.d.y >= 0) nd.d.y = static_cast<int>(rank[nd.d.y]);
   out[s] = nd;
   out_parent[s] = i == 0 ? -1 : static_cast<int>(rank[parent[i]]);
-  out_reach[s] = 1;
 }
 
 // Step 7.
@@ -1136,7 +1134,7 @@ hipError_t build_wide(rmh_map* m, hipStream_t stream) {
 }  // namespace
 
 // Writes the n_reach reachable nodes of the ni radix-tree slots (root at slot 0; size =
-// interior nodes of the final tree per subtree), their parents and reach flags in preorder
+// interior nodes of the final tree per subtree) and their parents in preorder
 // into the map's tree block.  rank and err are scratch.
 static hipError_t preorder_nodes(rmh_map* m, uint32_t ni, uint32_t n_reach, const Node2* nodes, const int* parent,
                                  const uint8_t* reach, const uint32_t* size, uint32_t* rank, uint32_t* err,
@@ -1146,7 +1144,6 @@ static hipError_t preorder_nodes(rmh_map* m, uint32_t ni, uint32_t n_reach, cons
     c.size = 0;
     m->nodes = c.take<Node2>(n_reach);
     m->parent = c.take<int>(n_reach);
-    m->reach = c.take<uint8_t>(n_reach);
     if (pass == 0) {
       const hipError_t e = hipMalloc(&m->tree_block, c.size);
       if (e != hipSuccess) { m->tree_block = nullptr; return e; }
@@ -1160,7 +1157,7 @@ static hipError_t preorder_nodes(rmh_map* m, uint32_t ni, uint32_t n_reach, cons
   }
   if (e == hipSuccess) {
     k_preorder_scatter<<<blocks_for(ni), kBlock, 0, stream>>>(ni, n_reach, reach, parent, nodes, rank, m->nodes,
-                                                              m->parent, m->reach, err);
+                                                              m->parent, err);
     e = hipGetLastError();
   }
   uint32_t herr = 0, root_size = 0;

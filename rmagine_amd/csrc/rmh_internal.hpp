@@ -156,7 +156,7 @@ struct RefitPass {
 struct rmh_map {
   uint32_t n_vertices = 0, n_faces = 0, n_meshes = 0;
   // device memory of the map: one block of the arrays whose sizes the mesh gives (vertices,
-  // faces, tris, normals), one of those the tree gives (nodes, parent, reach); freeing seven
+  // faces, tris, normals), one of those the tree gives (nodes, parent); freeing seven
   // arrays one by one took 1.4 ms for 2.1M triangles
   void* mesh_block = nullptr;
   void* tree_block = nullptr;
@@ -171,7 +171,6 @@ struct rmh_map {
   int device = 0;
   std::vector<uint32_t> mesh_offsets;  // host copy: faces of mesh g are [off[g], off[g+1])
   int* parent = nullptr;               // parent of each interior node (refit), -1 at the root
-  uint8_t* reach = nullptr;            // 1 for the interior nodes of the final tree
   // 4-wide quantised tree collapsed from the binary one; the ray kernels traverse it when
   // present (nodes4 != NULL), closest-point queries and refit work on the binary tree
   rmh::Node4* nodes4 = nullptr;
