@@ -39,11 +39,17 @@ def _ptr(t) -> ctypes.c_void_p:
     return ctypes.c_void_p(0 if t is None else int(t.data_ptr()))
 
 
+# a private function of torch, absent from builds without a GPU backend
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_handle(stream=None) -> ctypes.c_void_p:
     # the current device's current stream without the Stream object that current_stream() makes
     # (2.9 -> 0.4 us of every call; registering one scan makes two)
     if stream is None:
-        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+        if _raw_stream is not None:
+            return ctypes.c_void_p(_raw_stream(torch.cuda.current_device()))
+        stream = torch.cuda.current_stream()
     return ctypes.c_void_p(int(stream.cuda_stream))
 
 
