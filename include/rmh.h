@@ -122,6 +122,10 @@ const char* rmh_last_error(void);
 int rmh_version(void);
 int rmh_get_device_count(int* count);
 int rmh_set_device(int device);
+/* Gives the memory that the library's scratch pools keep between calls (closest-point queries and
+ * BVH builds; at most 1 GiB per device) back to the driver.  Memory of calls that have not
+ * finished stays; later calls take what they need again. */
+int rmh_release_scratch(void);
 int rmh_malloc(void** ptr_dev, size_t bytes);
 int rmh_free(void* ptr_dev);
 /* kind: 0 host->device, 1 device->host, 2 device->device, 3 host->host.  Blocking, like

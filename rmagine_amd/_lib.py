@@ -38,6 +38,7 @@ _SIGNATURES = {
     "rmh_version": (c_int, []),
     "rmh_get_device_count": (c_int, [ctypes.POINTER(c_int)]),
     "rmh_set_device": (c_int, [c_int]),
+    "rmh_release_scratch": (c_int, []),
     "rmh_malloc": (c_int, [ctypes.POINTER(c_void_p), c_size]),
     "rmh_free": (c_int, [c_void_p]),
     "rmh_memcpy": (c_int, [c_void_p, c_void_p, c_size, c_int]),

@@ -32,14 +32,17 @@ int hip_fail(hipError_t e, const char* what) {
   return RMH_ERR_HIP;
 }
 
+namespace {
+constexpr int kMaxPoolDevices = 64;
+std::mutex pools_mu;
+hipMemPool_t pools[kMaxPoolDevices] = {};
+}  // namespace
+
 // With the default pool, whose memory is returned and mapped again around every
 // synchronisation, sorting 4M queries paid 0.3 ms more per call.
 hipMemPool_t scratch_pool(int device) {
-  constexpr int kMaxPoolDevices = 64;
-  static std::mutex mu;
-  static hipMemPool_t pools[kMaxPoolDevices] = {};
   if (device < 0 || device >= kMaxPoolDevices) return nullptr;
-  std::lock_guard<std::mutex> lock(mu);
+  std::lock_guard<std::mutex> lock(pools_mu);
   if (!pools[device]) {
     hipMemPoolProps props = {};
     props.allocType = hipMemAllocationTypePinned;
@@ -73,6 +76,13 @@ int rmh_get_device_count(int* count) {
 
 int rmh_set_device(int device) {
   RMH_HIP_TRY(hipSetDevice(device));
+  return RMH_OK;
+}
+
+int rmh_release_scratch(void) {
+  std::lock_guard<std::mutex> lock(pools_mu);
+  for (hipMemPool_t p : pools)
+    if (p) RMH_HIP_TRY(hipMemPoolTrimTo(p, 0));
   return RMH_OK;
 }
 

@@ -53,6 +53,12 @@ def stream_handle(stream=None) -> ctypes.c_void_p:
     return ctypes.c_void_p(int(stream.cuda_stream))
 
 
+def release_scratch() -> None:
+    """Gives the device memory that librmh keeps between calls for closest-point queries and BVH
+    builds (at most 1 GiB per device) back to the driver; synchronise first."""
+    _lib.call("rmh_release_scratch")
+
+
 def _device_tensor(x, dtype, device) -> torch.Tensor:
     if isinstance(x, torch.Tensor):
         return x.to(device=device, dtype=dtype).contiguous()
