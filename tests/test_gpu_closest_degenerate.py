@@ -49,3 +49,25 @@ def test_queries_around_a_degenerate_triangle(shape, max_distance):
             continue
         np.testing.assert_allclose(dist[i], np.sqrt(least), rtol=2e-7, atol=1e-7)
         assert d2[face[i]] <= least * (1 + 1e-9) + 1e-14
+
+
+def test_meshes_of_thin_triangles():
+    """Every triangle without FP32 bounds: a fan around a vertex and scattered needles."""
+    rng = np.random.default_rng(12)
+    a = np.linspace(0, 2 * np.pi, 2500, endpoint=False)
+    fan = np.concatenate([[[0, 0, 0]], np.stack([5 * np.cos(a), 5 * np.sin(a), 0.01 * np.sin(7 * a)], 1)])
+    i = np.arange(2500)
+    Ff = np.stack([0 * i, i + 1, (i + 1) % 2500 + 1], 1)
+    at, d = rng.uniform(-5, 5, (400, 1, 3)), rng.normal(size=(400, 1, 3))
+    thin = at + np.array([0, 1, 0.5])[None, :, None] * d + np.array([0, 0, 2e-4])[None, :, None] * rng.normal(size=(400, 3, 3))
+    V = np.concatenate([fan, thin.reshape(-1, 3)]).astype(np.float32)
+    F = np.concatenate([Ff, np.arange(1200).reshape(-1, 3) + len(fan)]).astype(np.uint32)
+    Q = rng.uniform(-6, 6, (400, 3)).astype(np.float32)
+    Q[::4, 2] = 0.0
+    r = HipMap(V, F).closest_points(torch.as_tensor(Q, device="cuda"))
+    dist, face = r["dist"].cpu().numpy(), r["face_ids"].cpu().numpy()
+    corners = [V.astype(np.float64)[F[:, j].astype(np.int64)] for j in range(3)]
+    for k, q in enumerate(Q.astype(np.float64)):
+        d2 = ((C.closest_on_triangles(q, *corners) - q) ** 2).sum(1)
+        np.testing.assert_allclose(dist[k], np.sqrt(d2.min()), rtol=2e-7, atol=1e-7)
+        assert d2[face[k]] <= d2.min() * (1 + 1e-9) + 1e-14
