@@ -48,13 +48,16 @@ constexpr int kWave = 64;
 // nodes around a pose in one L2, but an XCD whose poses are dear ends late: over a deep map
 // with few poses, or where a pose's cost varies several times (a camera looks at much or at
 // nothing), runs of 256 rays are dealt to the XCDs in turn instead.
-// Microseconds, contiguous / dealt: 60 and 200 cameras of 640x480 1,930 / 1,629 and 5,798 /
-// 5,246; 30 lidars of 128 x 1,024 on 2.1M triangles 693 / 586, 100 of them 1,140 / 1,133, 250
-// of them 2,234 / 2,273.  Casts in rooms, whose map fits every L2, gain or lose: 12 lidars of
-// 64 x 1,024 77.3 / 72.0, 18 of 20 x 714 68.8 / 71.3, 100 VLP-16 106.9 / 111.0, 320 x 240 cameras, 8 poses
-// 53.7 / 56.8, 30 poses 111.2 / 102.5: they stay contiguous.  Scattered lists, of
-// which every XCD would write a part of each output line, lose (256 lists of 32,768 rays from
-// one place, points, normals and hits: 2,530 / 2,690; 30 lists of 20,000 in a room 90 / 100).
+// Microseconds, contiguous / dealt, on maps of 500,000 triangles or more: 60 and 200 cameras of
+// 640x480 1,930 / 1,629 and 5,798 / 5,246; 30 lidars of 128 x 1,024 on 2.1M triangles 693 / 586, 100 of them 1,140 / 1,133, 250
+// of them 2,234 / 2,273: the line at 64 poses gives up the 0.6 % of 100.  Casts in rooms of at
+// most 25,000 triangles, whose map fits every L2, gain or lose: 12 lidars of 64 x 1,024
+// 77.3 / 72.0, 30 VLP-16 87 / 82, 18 lidars of 20 x 714 68.8 / 71.3, 100 VLP-16 106.9 / 111.0,
+// 320 x 240 cameras, 8 poses 53.7 / 56.8, 30 poses 111.2 / 102.5.  No rule of sizes separates
+// them, so they keep the contiguous order.  Nothing between 50,000 and 500,000 triangles was
+// measured to place kDeepMap.  Scattered lists, of which every XCD would write a part of each
+// output line, lose (256 lists of 32,768 rays from one place, points, normals and hits:
+// 2,530 / 2,690; 30 lists of 20,000 in a room 90 / 100).
 constexpr uint32_t kWholePoses = 64, kDealRays = 256;
 
 struct SimArgs {
@@ -69,7 +72,7 @@ struct SimArgs {
 };
 
 // Launch bounds ask for 8 waves per SIMD (64 VGPRs); with the writers' values recomputed or
-// re-read after the traversal, nothing spills (62-64 VGPRs, 62 SGPRs).
+// re-read after the traversal, one or two VGPRs spill (64 VGPRs, 62-66 SGPRs).
 template <int KIND, int STACK, bool WIDE, int SPEC>
 __global__ __launch_bounds__(kWave, 8) void k_simulate(const SimArgs a) {
   __shared__ int2 stk[kLdsStack][kWave];
