@@ -200,5 +200,6 @@ struct rmh_sensor {
   uint32_t* perm = nullptr;
   int sorted = 1;                 // traversal order: RMH_RAY_ORDER_LIST / _SORTED / _TILES
   int speculative = 1;            // O1Dn / OnDn walk in rmh_simulate: speculative or classic
+  int scattered = 0;              // O1Dn / OnDn: the rays of a wave point apart, in traversal order
   int device = 0;
 };

@@ -239,6 +239,43 @@ __global__ void k_gather_rays(const uint32_t* __restrict__ order, uint32_t n, co
   if (o_in) o_out[s] = o_in[i];
 }
 
+// Sum over the runs of 64 rays of 1 - |mean unit direction|, 0 where a run's rays are parallel,
+// near 1 where they point everywhere.
+__global__ __launch_bounds__(64) void k_run_spread(const rmh_vec3* __restrict__ d, uint32_t n, float* __restrict__ sum) {
+  const uint32_t base = blockIdx.x * 64u, i = base + threadIdx.x, cnt = n - base < 64u ? n - base : 64u;
+  float x = 0.0f, y = 0.0f, z = 0.0f;
+  if (i < n) {
+    const rmh_vec3 v = d[i];
+    const float l2 = v.x * v.x + v.y * v.y + v.z * v.z;
+    const float r = l2 > 0.0f && l2 < INFINITY ? 1.0f / sqrtf(l2) : 0.0f;
+    x = v.x * r; y = v.y * r; z = v.z * r;
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    x += __shfl_xor(x, off, 64);
+    y += __shfl_xor(y, off, 64);
+    z += __shfl_xor(z, off, 64);
+  }
+  if (threadIdx.x == 0) atomicAdd(sum, 1.0f - sqrtf(x * x + y * y + z * z) / static_cast<float>(cnt));
+}
+
+// Whether the rays that a wave casts together (runs of 64 in traversal order) point apart: a mean
+// of 0.3 is a half angle of about 45 degrees (a 16 x 900 scanner's tiles 0.004, random rays 0.88).
+static hipError_t runs_scattered(const rmh_sensor* s, uint32_t n, int* scattered) {
+  const uint32_t runs = n / 64u + (n % 64u != 0u);
+  float* sum = nullptr;
+  float h = 0.0f;
+  hipError_t e = hipMalloc(&sum, sizeof(float));
+  if (e == hipSuccess) e = hipMemset(sum, 0, sizeof(float));
+  if (e == hipSuccess) {
+    k_run_spread<<<runs, 64>>>(s->dirs, n, sum);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) e = hipMemcpy(&h, sum, sizeof(float), hipMemcpyDeviceToHost);
+  if (sum) (void)hipFree(sum);
+  *scattered = h > 0.3f * static_cast<float>(runs) ? 1 : 0;
+  return e;
+}
+
 // Uploads n rays (device pointers from the caller) into s->dirs / s->origs in direction
 // order and fills s->order.  Blocking (sensor creation is not on a timed path).
 static hipError_t upload_sorted_rays(rmh_sensor* s, const rmh_vec3* dirs_in, const rmh_vec3* origs_in, uint32_t n) {
@@ -270,6 +307,7 @@ static hipError_t upload_sorted_rays(rmh_sensor* s, const rmh_vec3* dirs_in, con
     k_gather_rays<<<blocks, 256>>>(s->order, n, dirs_in, origs_in, s->dirs, s->origs);
     e = hipGetLastError();
   }
+  if (e == hipSuccess) e = runs_scattered(s, n, &s->scattered);
   if (e == hipSuccess) e = hipDeviceSynchronize();
   s->sorted = 1;
   if (keys) (void)hipFree(keys);
@@ -301,6 +339,7 @@ int rmh_sensor_set_ray_order(rmh_sensor* s, int order) {
   }
   k_gather_rays<<<blocks, 256>>>(s->order, n, s->dirs_list, s->origs_list, s->dirs, s->origs);
   RMH_HIP_TRY(hipGetLastError());
+  RMH_HIP_TRY(runs_scattered(s, n, &s->scattered));
   RMH_HIP_TRY(hipDeviceSynchronize());
   s->sorted = order;
   return RMH_OK;

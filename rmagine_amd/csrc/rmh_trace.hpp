@@ -643,7 +643,8 @@ constexpr uint32_t kDefaultTileRows = 4;
 // the chip's 8,192 wave slots are empty.  Rays are split over more waves as long as half a
 // round of waves results; on a deep map (kDeepMap triangles or more: long walks, whose rays
 // differ most) two rounds, or for scattered lists (whose waves are long and uneven at any
-// size) 5/8 of one.  Measured, microseconds, 64 rays -> the rule's choice: 16 x 900 lidar in a
+// size: those walked speculatively, and grids whose tiles hold rays that point apart, which two
+// rounds made 15-43 % slower at 65,000 to 520,000 rays) 5/8 of one.  Measured, microseconds, 64 rays -> the rule's choice: 16 x 900 lidar in a
 // room (2,412 triangles) 1 pose 49 -> 36 (4 rays), 4 poses 54 -> 50 (16), 16 poses 63 (32 rays 62,
 // 16 rays 74; in a room of 25k triangles 48, 50 and 61); the lidar on 500k triangles 144 -> 65
 // (2); 128 x 1,024 lidar on 2.1M triangles 1 pose 222 -> 149 (8), 4 poses 358 -> 296 (32); 640 x 480
