@@ -11,7 +11,8 @@
 // bound of its distance, the upper ones shrink the search, and the triangles whose lower
 // bound does not exceed it are listed.  The list (6 slots per lane in LDS, emptied when a
 // closer triangle outdates all of it) is evaluated in FP64 at the end, when all lanes are
-// there, or when it is full: the triangle's closest point (Ericson, Real-Time Collision
+// there, or when it is full or takes a degenerate triangle or sliver, which have no bounds: the
+// triangle's closest point (Ericson, Real-Time Collision
 // Detection, 5.1.5: Voronoi regions of the vertices, edges and face) and its distance, so the
 // result is the FP64 nearest triangle; equal distances go to the lower global face index.
 // Evaluated in the leaves, the FP64 code ran for nearly every triangle, for one or two lanes
