@@ -11,8 +11,8 @@
 // bound of its distance, the upper ones shrink the search, and the triangles whose lower
 // bound does not exceed it are listed.  The list (6 slots per lane in LDS, emptied when a
 // closer triangle outdates all of it) is evaluated in FP64 at the end, when all lanes are
-// there, or when it is full or takes a degenerate triangle or sliver, which have no bounds: the
-// triangle's closest point (Ericson, Real-Time Collision
+// there, or when a triangle is to be listed and it is full or ends with a degenerate triangle or
+// sliver, which have no bounds: the triangle's closest point (Ericson, Real-Time Collision
 // Detection, 5.1.5: Voronoi regions of the vertices, edges and face) and its distance, so the
 // result is the FP64 nearest triangle; equal distances go to the lower global face index.
 // Evaluated in the leaves, the FP64 code ran for nearly every triangle, for one or two lanes
@@ -108,6 +108,7 @@ __global__ __launch_bounds__(64, 5) void k_closest(const CPArgs a) {
   float bound = walk_bound(upper);      // boxes beyond it hold nothing nearer
   float least = __builtin_inff();       // least lower bound of the listed triangles
   uint32_t n_cand = 0;
+  bool thin = false;                    // the last listed triangle has no upper bound
   auto evaluate = [&]() {
     const D3 q = d3(qv.x, qv.y, qv.z);
     for (uint32_t k = 0; k < n_cand; k++) {
@@ -144,19 +145,22 @@ __global__ __launch_bounds__(64, 5) void k_closest(const CPArgs a) {
         upper = d.hi;
         if (upper < least) { n_cand = 0; least = __builtin_inff(); }
       }
-      cand[n_cand][threadIdx.x] = first + k;
-      n_cand++;
-      least = fminf(least, d.lo);
-      // A triangle without an upper bound shrinks the search by its FP64 distance, at once: left in
-      // the list, it did so only when the list overflowed, lane by lane (200,000 queries around a
-      // fan of 3,000 thin triangles 13.7 ms, 8.2 so, 7.4 with every triangle in FP64; a fan of
-      // 100,000 528, 308 and 317; 50,000 needles 0.21, 0.20 and 0.24.  Asking for the shape before
-      // the bounds are formed brings the first to 6.8 ms, but 1M terrain queries to 1.87 or 1.92 ms
-      // from 1.81).
-      if (n_cand == kCand || !(d.hi < __builtin_inff())) {
+      // A triangle without an upper bound shrinks the search by its FP64 distance when the next
+      // one is listed; left in the list, it did so only when the list overflowed, lane by lane
+      // (200,000 queries around a fan of 3,000 thin triangles 13.5 ms, 7.9 so, 7.4 with every
+      // triangle in FP64; a fan of 100,000 529, 313 and 313; 50,000 needles 0.21, 0.22 and 0.23).
+      // Evaluated as it is listed, which fills the list at six: fan 8.2 ms, but 200,000 to
+      // 600,000 queries in a room of 50k triangles 8 % slower; at the end of the leaf, in code of
+      // its own: small batches 2-5 % slower; with the shape asked for before the bounds are
+      // formed: fan 6.8 ms, but 1M terrain queries 3-6 % slower.
+      if (n_cand == kCand || thin) {
         evaluate();
         upper = fminf(upper, upper_f32(best));
       }
+      cand[n_cand][threadIdx.x] = first + k;
+      n_cand++;
+      least = fminf(least, d.lo);
+      thin = !(d.hi < __builtin_inff());
     }
     bound = walk_bound(upper);
   };
@@ -174,6 +178,12 @@ __global__ __launch_bounds__(64, 5) void k_closest(const CPArgs a) {
       g = b0 <= b1 ? nd.d.x : nd.d.y;
     }
     leaf_test(g);
+    if (thin) {  // a bound from slivers too: without it 50,000 needles take 0.27 ms
+      evaluate();
+      upper = fminf(upper, upper_f32(best));
+      bound = walk_bound(upper);
+      thin = false;
+    }
     n_cand = 0;  // the walk meets that leaf again
     least = __builtin_inff();
     ref = a.map.root;
